@@ -37,9 +37,9 @@ struct gse_handle {
   double *qmax = nullptr;             // [max_rows][nsl]
   gse::Fx *qpart = nullptr;           // [max_rows][nsl]
   gse::QFin *qfin = nullptr;          // [max_rows]
-  double *pmax = nullptr;             // [max_rows][nsl]
+  double *pmax = nullptr;             // [max_rows][2 nsl]
   gse::Fx *ppart = nullptr;           // [max_rows][nsl]
-  int32_t *plast = nullptr;           // [max_rows][nsl]
+  int32_t *plast = nullptr;           // [max_rows][2 nsl]
   uint64_t *ptop = nullptr;           // [max_rows][nsl][4 * GSE_MAX_KIDS]
   uint32_t *ptick = nullptr;
   uint32_t *plist = nullptr;          // [GSE_MAX_KIDS + 1][max_rows] nodes of each verify residual pass
@@ -261,6 +261,18 @@ void carve(gse_handle *h, void *block, const gse::Layout &L, bool tree) {
   h->pcnt = (uint32_t *)(b + L.pcnt);
 }
 
+// The row passes' view of the handle's workspace (gse_rows.hip).
+gse::RowsWs rows_ws(const gse_handle *h) {
+  gse::RowsWs w;
+  w.rows = (int)h->max_rows;
+  w.slices = (int)(h->nsl * (gse::CH / gse::RS));
+  w.sum = h->pmax;
+  w.seg = (double *)h->tseg;
+  w.last = h->plast;
+  w.tick = h->ptick;
+  w.st = h->tstate;
+  return w;
+}
 
 // ---- the static workspace of gse_sample_noalloc --------------------------------------------------------------------
 // One per GPU: a file-scope device array (each device holds its own copy from the library's load until the process
@@ -547,7 +559,7 @@ GSE_API int gse_draw(gse_handle *h, const double *q, int64_t q_ld, uint32_t rows
   if (vocab == 0 || q_ld < (int64_t)vocab) return fail(h, GSE_E_ARG, "vocab 0 or q_ld < vocab");
   if (rows == 0) return GSE_OK;
   DeviceGuard g(h->device);
-  hipError_t e = gse::launch_draw(q, q_ld, (int)rows, (int)vocab, u, out, (hipStream_t)stream);
+  hipError_t e = gse::launch_draw(rows_ws(h), q, q_ld, (int)rows, (int)vocab, u, out, (hipStream_t)stream);
   return e == hipSuccess ? GSE_OK : hip_fail(h, e, "draw launch");
 }
 
@@ -561,7 +573,7 @@ GSE_API int gse_mss(gse_handle *h, const gse_mss_batch *in) {
   if (b.q && b.q_ld < (int64_t)b.vocab) return fail(h, GSE_E_ARG, "q_ld < vocab");
   if (b.nodes == 0) return GSE_OK;
   DeviceGuard g(h->device);
-  hipError_t e = gse::launch_mss(b, (hipStream_t)b.stream);
+  hipError_t e = gse::launch_mss(rows_ws(h), b, (hipStream_t)b.stream);
   return e == hipSuccess ? GSE_OK : hip_fail(h, e, "mss launch");
 }
 

@@ -197,6 +197,17 @@ struct TreeLaunch {
   gse_tree_out out;
 };
 
+// The workspace of the row passes (gse_rows.hip): per row, `slices` slices of RS tokens.
+constexpr int RS = 4096;
+struct RowsWs {
+  int rows, slices;
+  double *sum;      // [rows][slices] slice sums
+  double *seg;      // [rows][slices][64] segment sums
+  int32_t *last;    // [rows][slices] last token with a positive weight
+  uint32_t *tick;   // [rows] slice tickets, zero between calls
+  TreeNode *st;     // [rows] state of a node between launches (its ticket zero between calls)
+};
+
 struct PickLaunch {
   gse_pick_batch b;
   double *pmax;
@@ -243,13 +254,14 @@ constexpr Layout plan_layout(uint32_t R, uint32_t V, uint32_t target, bool tree)
     L.tstate = put((size_t)R * sizeof(TreeNode));
     L.npart = put((size_t)R * K * S * sizeof(Fx));
     L.nlast = put((size_t)R * K * S * sizeof(int32_t));
-    L.tseg = put((size_t)R * S * 2 * (CH / 64) * sizeof(uint64_t));  // the last residual's 64-token segment sums
+    L.tseg = put((size_t)R * S * 2 * (CH / 64) * sizeof(uint64_t));  // the last residual's 64-token segment sums; or
+                                                                     // the row passes' segment sums
     L.qmax = put((size_t)R * S * sizeof(double));
     L.qpart = put((size_t)R * S * sizeof(Fx));
     L.qfin = put((size_t)R * sizeof(QFin));
-    L.pmax = put((size_t)R * S * sizeof(double));
+    L.pmax = put((size_t)R * S * (CH / RS) * sizeof(double));
     L.ppart = put((size_t)R * S * sizeof(Fx));
-    L.plast = put((size_t)R * S * sizeof(int32_t));
+    L.plast = put((size_t)R * S * (CH / RS) * sizeof(int32_t));
     L.ptop = put((size_t)R * S * 4 * GSE_MAX_KIDS * sizeof(uint64_t));
     L.ptick = put((size_t)R * sizeof(uint32_t));
     L.plist = put((size_t)(GSE_MAX_KIDS + 1) * R * sizeof(uint32_t));  // the nodes of each residual pass
@@ -263,8 +275,10 @@ hipError_t launch_main(const ScanArgs &a, hipStream_t s);
 hipError_t launch_deep(const ScanArgs &a, hipStream_t s);
 hipError_t launch_exact(const ScanArgs &a, hipStream_t s);
 hipError_t launch_dist_write(const ScanArgs &a, double *probs, int64_t probs_ld, hipStream_t s);
-hipError_t launch_draw(const double *q, int64_t ld, int rows, int V, const double *u, int32_t *out, hipStream_t s);
-hipError_t launch_mss(const gse_mss_batch &b, hipStream_t s);
+// Row passes (gse_rows.hip): draw() and mss() over fp64 rows.
+hipError_t launch_draw(const RowsWs &w, const double *q, int64_t ld, int rows, int V, const double *u, int32_t *out,
+                       hipStream_t s);
+hipError_t launch_mss(const RowsWs &w, const gse_mss_batch &b, hipStream_t s);
 // The verify round after the selection pass (the statistics of the q rows given as drafter logits included).
 hipError_t launch_tree(const TreeLaunch &L, hipStream_t s);
 hipError_t launch_pick(const PickLaunch &L, hipStream_t s);

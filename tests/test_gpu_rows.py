@@ -1,0 +1,110 @@
+"""GPU parity of the row passes (draw, mss) at the edges of their slices and segments, against the oracle: tokens and
+accepted kids are compared exactly (a draw within rounding of a prefix boundary has a probability of about 1e-13)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import sampling_ref as ora
+from oracle import spec_ref as spo
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 2, 63, 64, 65, 4095, 4096, 4097, 50257, 262147]
+
+
+@pytest.mark.parametrize("v", SIZES)
+def test_draw_sizes(ge, gpu, v):
+    """Positive rows, sparse rows (long zero runs before, between and after the mass) and u at 0 and just below 1."""
+    rng = np.random.default_rng(v)
+    for kind in range(3):
+        q = rng.random(v)
+        if kind == 1:
+            q[rng.random(v) < 0.999] = 0.0
+            q[rng.integers(0, v)] = 0.5
+        if kind == 2:
+            q[:] = 0.0
+            q[v // 2] = 1.0
+        qt = torch.from_numpy(q).to(gpu)
+        for u in [0.0, 0.3, 0.9, 1.0 - 2.0 ** -53]:
+            assert ge.sampling.draw(qt, u) == ora.draw(q, u), (v, kind, u)
+    with pytest.raises(IndexError):
+        ge.sampling.draw(torch.zeros(v, dtype=torch.float64, device=gpu), 0.5)
+
+
+def _nodes(v, n, rng):
+    """Nodes of 0 .. 5 kids over [n, v] targets: kids with a distribution of their own, kids sharing one, one-hot kids;
+    the kids' tokens are where q most exceeds p, so that most are rejected and the deeper levels run."""
+    p = rng.random((n, v)) ** 4
+    p[:, rng.random(v) < 0.3] = 0.0
+    p[:, 0] += 1e-3
+    p /= p.sum(1, keepdims=True)
+    kids = []
+    for a in range(n):
+        q = [rng.random(v) ** 4 for _ in range(2)]
+        q = [x / x.sum() for x in q]
+        ks = []
+        for r in range(a % 6):
+            if (a + r) % 4 == 3:
+                ks.append((int(rng.integers(0, v)), None))
+            else:
+                j = (a + r) % 2
+                ks.append((int(np.argsort(p[a] - q[j])[min(r, v - 1)]), q[j]))
+        kids.append(ks)
+    return p, kids
+
+
+@pytest.mark.parametrize("v", SIZES)
+def test_mss_sizes(ge, gpu, v):
+    n = 12 if v < 100000 else 6
+    p, kids = _nodes(v, n, np.random.default_rng(v))
+    levels = set()
+    for seed in range(3):
+        toks, ks = ge.spec.mss_batch(torch.from_numpy(p).to(gpu), kids, [seed * 100 + a for a in range(n)], [5] * n)
+        for a in range(n):
+            want = spo.mss(p[a], kids[a], seed * 100 + a, 5)
+            assert (toks[a], ks[a]) == want, (v, seed, a)
+            levels.add(len(kids[a]) if want[1] is None else want[1])
+    if v >= 63:
+        assert max(levels) == 5, levels  # a node whose five kids were all rejected
+
+
+def test_rows_past_the_handles_size(ge, gpu):
+    """A handle opened for one row of 64 tokens serves draw and mss over more rows of a longer vocabulary: its few
+    slices widen and the rows go out in several launches."""
+    lib = ge._lib
+    h = lib.Handle(gpu.index, 1, 64)
+    rng = np.random.default_rng(3)
+    v, rows = 50257, 5
+    q = rng.random((rows, v)) * (rng.random((rows, v)) < 0.5)
+    u = rng.random(rows)
+    qd, ud = torch.from_numpy(q).to(gpu), torch.from_numpy(u).to(gpu)
+    out = torch.full((rows,), -7, dtype=torch.int32, device=gpu)
+    for _ in range(2):
+        h.call("gse_draw", qd.data_ptr(), v, rows, v, ud.data_ptr(), out.data_ptr(), lib.stream_of(gpu.index))
+        assert out.cpu().tolist() == [ora.draw(q[r], u[r]) for r in range(rows)]
+    p, kids = _nodes(v, 6, rng)
+    kmax = 5
+    kt, kq, qs = np.full((6, kmax), -1, np.int32), np.full((6, kmax), -1, np.int32), []
+    for a, ks in enumerate(kids):
+        for r, (x, qq) in enumerate(ks):
+            kt[a, r] = x
+            if qq is not None:
+                kq[a, r] = len(qs)
+                qs.append(qq)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu)  # noqa: E731
+    pd, qd, ktd, kqd = dev(p), dev(np.stack(qs)), dev(kt), dev(kq)
+    sd, ix = dev(np.arange(6, dtype=np.int64) + 40), dev(np.full(6, 9, np.int64))
+    ot, ok = torch.empty(6, dtype=torch.int32, device=gpu), torch.empty(6, dtype=torch.int32, device=gpu)
+    b = lib.MssBatch()
+    b.size, b.nodes, b.vocab, b.max_kids = C.sizeof(lib.MssBatch), 6, v, kmax
+    b.p, b.p_ld, b.q, b.q_ld = pd.data_ptr(), v, qd.data_ptr(), v
+    b.kid_tok, b.kid_q, b.seed, b.idx = ktd.data_ptr(), kqd.data_ptr(), sd.data_ptr(), ix.data_ptr()
+    b.out_token, b.out_kid = ot.data_ptr(), ok.data_ptr()
+    b.stream = torch.cuda.current_stream(gpu).cuda_stream
+    h.call("gse_mss", C.byref(b))
+    want = [spo.mss(p[a], kids[a], 40 + a, 9) for a in range(6)]
+    assert ot.cpu().tolist() == [t for t, _ in want]
+    assert ok.cpu().tolist() == [-1 if r is None else r for _, r in want]
+    h.close()
