@@ -38,9 +38,9 @@ struct gse_handle {
   gse::Fx *qpart = nullptr;           // [max_rows][nsl]
   gse::QFin *qfin = nullptr;          // [max_rows]
   double *pmax = nullptr;             // [max_rows][2 nsl]
-  gse::Fx *ppart = nullptr;           // [max_rows][nsl]
+  gse::Fx *ppart = nullptr;           // [max_rows][2 nsl]
   int32_t *plast = nullptr;           // [max_rows][2 nsl]
-  uint64_t *ptop = nullptr;           // [max_rows][nsl][4 * GSE_MAX_KIDS]
+  uint64_t *ptop = nullptr;           // [max_rows][2 nsl][GSE_MAX_KIDS]
   uint32_t *ptick = nullptr;
   uint32_t *plist = nullptr;          // [GSE_MAX_KIDS + 1][max_rows] nodes of each verify residual pass
   uint32_t *pcnt = nullptr;           // [GSE_MAX_KIDS + 1]          // [max_rows]
@@ -266,10 +266,13 @@ gse::RowsWs rows_ws(const gse_handle *h) {
   gse::RowsWs w;
   w.rows = (int)h->max_rows;
   w.slices = (int)(h->nsl * (gse::CH / gse::RS));
+  w.round = (int)h->target;
   w.sum = h->pmax;
   w.seg = (double *)h->tseg;
   w.last = h->plast;
   w.tick = h->ptick;
+  w.mass = h->ppart;
+  w.top = h->ptop;
   w.st = h->tstate;
   return w;
 }
@@ -525,14 +528,7 @@ GSE_API int gse_draft_pick(gse_handle *h, const gse_pick_batch *in) {
   if (b.vocab > h->max_vocab)
     return fail(h, GSE_E_CAPACITY, "vocab %u, the handle was opened for %u", b.vocab, h->max_vocab);
   DeviceGuard g(h->device);
-  gse::PickLaunch L = {};
-  L.b = b;
-  L.pmax = h->pmax;
-  L.ppart = h->ppart;
-  L.plast = h->plast;
-  L.ptop = h->ptop;
-  L.tick = h->ptick;
-  hipError_t e = gse::launch_pick(L, (hipStream_t)b.stream);
+  hipError_t e = gse::launch_pick(rows_ws(h), b, (hipStream_t)b.stream);
   return e == hipSuccess ? GSE_OK : hip_fail(h, e, "pick launch");
 }
 

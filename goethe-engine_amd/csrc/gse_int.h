@@ -201,20 +201,14 @@ struct TreeLaunch {
 constexpr int RS = 4096;
 struct RowsWs {
   int rows, slices;
+  int round;        // workgroups of one resident round (four per CU)
   double *sum;      // [rows][slices] slice sums
   double *seg;      // [rows][slices][64] segment sums
   int32_t *last;    // [rows][slices] last token with a positive weight
   uint32_t *tick;   // [rows] slice tickets, zero between calls
+  Fx *mass;         // [rows][slices] slice masses
+  uint64_t *top;    // [rows][slices][GSE_MAX_KIDS] the slices' best entries
   TreeNode *st;     // [rows] state of a node between launches (its ticket zero between calls)
-};
-
-struct PickLaunch {
-  gse_pick_batch b;
-  double *pmax;
-  Fx *ppart;
-  int32_t *plast;
-  uint64_t *ptop;
-  uint32_t *tick;
 };
 
 // Byte layout of a device workspace for max_rows x max_vocab; target: main-pass workgroups to aim for (4 per CU).
@@ -260,9 +254,9 @@ constexpr Layout plan_layout(uint32_t R, uint32_t V, uint32_t target, bool tree)
     L.qpart = put((size_t)R * S * sizeof(Fx));
     L.qfin = put((size_t)R * sizeof(QFin));
     L.pmax = put((size_t)R * S * (CH / RS) * sizeof(double));
-    L.ppart = put((size_t)R * S * sizeof(Fx));
+    L.ppart = put((size_t)R * S * (CH / RS) * sizeof(Fx));
     L.plast = put((size_t)R * S * (CH / RS) * sizeof(int32_t));
-    L.ptop = put((size_t)R * S * 4 * GSE_MAX_KIDS * sizeof(uint64_t));
+    L.ptop = put((size_t)R * S * (CH / RS) * GSE_MAX_KIDS * sizeof(uint64_t));
     L.ptick = put((size_t)R * sizeof(uint32_t));
     L.plist = put((size_t)(GSE_MAX_KIDS + 1) * R * sizeof(uint32_t));  // the nodes of each residual pass
     L.pcnt = put((GSE_MAX_KIDS + 1) * sizeof(uint32_t));
@@ -275,13 +269,13 @@ hipError_t launch_main(const ScanArgs &a, hipStream_t s);
 hipError_t launch_deep(const ScanArgs &a, hipStream_t s);
 hipError_t launch_exact(const ScanArgs &a, hipStream_t s);
 hipError_t launch_dist_write(const ScanArgs &a, double *probs, int64_t probs_ld, hipStream_t s);
-// Row passes (gse_rows.hip): draw() and mss() over fp64 rows.
+// Row passes (gse_rows.hip): draw() and mss() over fp64 rows, the drafter's picks.
 hipError_t launch_draw(const RowsWs &w, const double *q, int64_t ld, int rows, int V, const double *u, int32_t *out,
                        hipStream_t s);
 hipError_t launch_mss(const RowsWs &w, const gse_mss_batch &b, hipStream_t s);
 // The verify round after the selection pass (the statistics of the q rows given as drafter logits included).
 hipError_t launch_tree(const TreeLaunch &L, hipStream_t s);
-hipError_t launch_pick(const PickLaunch &L, hipStream_t s);
+hipError_t launch_pick(const RowsWs &w, const gse_pick_batch &b, hipStream_t s);
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
 hipError_t launch_qprob(const gse_qrows &q, int V, double *out, int64_t ld, hipStream_t s);
 hipError_t launch_pack(const uint8_t *bools, int64_t bld, int rows, int V, int32_t *words, int64_t wld, hipStream_t s);

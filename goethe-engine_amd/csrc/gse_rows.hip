@@ -5,11 +5,14 @@
 //
 //   draw  sampling.py:100-104  inverse CDF in vocabulary order of fp64 rows
 //   mss   spec.py:88-103       multi-step speculative sampling: one launch per residual level, at most MSS_LEVELS of them
+//   pick  spec.py:151-159      the drafter's children (TreeDrafter._pick) of rows of logits, one launch
 //
 // What bounds them: a slice is one round of coalesced 512-byte reads per wave (16 tokens a thread), so at the sizes of a
 // decode step a launch is latency: load, sums, ticket, the last slice's reads. One workgroup per row, each thread summing
 // a contiguous run (128 tokens at V = 128256: every load of a wave touched 64 cache lines, one CU per row), took 0.9 ms
 // for 16 mss nodes of V = 128256 and two kids, 85 % of a dist + mss call (1014 us); sliced, that call takes 106 us.
+#include <type_traits>
+
 #include "gse_dev.h"
 #include "gse_int.h"
 
@@ -382,6 +385,391 @@ __global__ __launch_bounds__(RT) void mss_kernel(MssArgs a) {
   if (tid == 0) mss_out(b, node, j, -1);
 }
 
+// ---- a slice of a row of logits in registers ---------------------------------------------------------------------------
+// Thread tid holds RE tokens of its slice: vector v of VEC consecutive tokens at s0 + (v RT + tid) VEC, so that a wave's
+// vector is one segment of 64 VEC tokens. Rows whose start is 16-byte aligned (AL) read whole vectors.
+constexpr int RE = RS / RT;
+template <int DT>
+struct RLay {
+  static constexpr int VEC = DT == GSE_BF16 ? 8 : 4, NV = RE / VEC, SEG = WAVE * VEC, NSEG = RS / SEG;
+};
+
+template <int DT, bool AL>
+__device__ __forceinline__ void load_vec(const char *base, int t0, int V, float *x) {
+  using L = RLay<DT>;
+  if (AL && t0 + L::VEC <= V) {
+    if constexpr (DT == GSE_BF16) {
+      const uint4 u = *reinterpret_cast<const uint4 *>(base + (size_t)t0 * 2);
+      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[2 * i] = __uint_as_float(w[i] << 16);
+        x[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
+      }
+    } else {
+      const float4 f = *reinterpret_cast<const float4 *>(base + (size_t)t0 * 4);
+      x[0] = f.x;
+      x[1] = f.y;
+      x[2] = f.z;
+      x[3] = f.w;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < L::VEC; ++e) {
+      const int t = min(t0 + e, V - 1);
+      float f;
+      if constexpr (DT == GSE_BF16) f = bf16_to_f32(((const uint16_t *)base)[t]);
+      else f = ((const float *)base)[t];
+      x[e] = t0 + e < V ? f : -INFINITY;
+    }
+  }
+}
+
+template <int DT>
+__device__ __forceinline__ double logit_at(const char *base, int t) {
+  if constexpr (DT == GSE_BF16) return (double)bf16_to_f32(((const uint16_t *)base)[t]);
+  else return (double)((const float *)base)[t];
+}
+
+// ---- pick: spec.py:151-159 -------------------------------------------------------------------------------------------
+// t > 0: n draws from softmax(x / t). A slice takes its own maximum m of z = x / t and the exact fixed-point masses
+// exp(z - m) of its segments in one read; the row's last slice scales the slices' masses by exp(m - M) (M the row's
+// maximum), in slice order, and its waves make the draws: crossing slice, crossing segment, crossing token.
+// t == 0: the n best in stable descending order. A wave's n-th largest lane maximum bounds its n-th largest element from
+// below, so the elements at or above it (n and a few) go to a list in LDS and are ranked by counting; the row's last
+// workgroup ranks the others' bests the same way. One launch: 64 bf16 rows of 128256 tokens,
+// n = 4, take 13.3 us (106 us with n rounds of a wave-wide 64-bit maximum over every element and a bitonic merge), two draws
+// of 32 f32 rows of 32000 tokens 11.6 us (45 us as three launches: maximum, masses, draws).
+constexpr uint64_t SALT_DRAFT = 1ull << 42;
+constexpr int TOPL = GSE_MAX_KIDS * RE;  // list entries of a wave, at most (n lanes of RE elements)
+
+struct PickArgs {
+  gse_pick_batch b;
+  int ns;
+  double *max;      // [rows][ns] slice maxima of z
+  Fx *mass, *seg;   // [rows][ns], [rows][ns][NSEG]: masses exp(z - slice maximum)
+  int32_t *last;    // [rows][ns] last token with a positive mass
+  uint64_t *top;    // [rows][ns][GSE_MAX_KIDS] packed (key, id), descending, 0 pads
+  uint32_t *tick;   // [rows]
+};
+
+struct PickShared {
+  union {
+    uint64_t list[RW][TOPL];
+    struct {
+      uint64_t shi[RW], slo[RW];
+      float mx[RW];
+      int last[RW];
+    } d;
+  };
+  uint64_t best[GSE_MAX_KIDS];
+  uint32_t cnt[RW];
+  uint32_t ticket;
+  double etab[64];
+};
+
+// The n-th largest of the lanes' packed keys (token ids below 2^21); 0 when fewer than n lanes hold one.
+__device__ __forceinline__ uint64_t wave_kth_packed(uint64_t v, int n) {
+  auto enough = [&](uint64_t c) { return (int)__popcll(ballot64(v >= c)) >= n; };
+  uint64_t r = 0;
+#pragma unroll 4
+  for (int b = 63; b >= 32; --b)
+    if (enough(r | 1ull << b)) r |= 1ull << b;
+  if (!enough(r | 0xFFE00000ull)) return 0ull;
+  r |= 0xFFE00000ull;
+#pragma unroll 4
+  for (int b = 20; b >= 0; --b)
+    if (enough(r | 1ull << b)) r |= 1ull << b;
+  return r;
+}
+
+// Ranks the waves' lists against each other: sh.best[0, n) = the n largest listed, descending (0 pads). c: this wave's
+// list length. Barriers before (the lists) and after.
+__device__ __forceinline__ void rank_lists(uint32_t c, int n, PickShared &sh) {
+  const int tid = threadIdx.x, w = tid >> 6;
+  if (lane_id() == 0) sh.cnt[w] = c;
+  if (tid < GSE_MAX_KIDS) sh.best[tid] = 0ull;
+  __syncthreads();
+  for (uint32_t i = lane_id(); i < c; i += WAVE) {
+    const uint64_t x = sh.list[w][i];
+    int r = 0;
+#pragma unroll 1
+    for (int q = 0; q < RW; ++q) {
+      const uint32_t m = sh.cnt[q];
+#pragma unroll 4
+      for (uint32_t j = 0; j < m; ++j) r += sh.list[q][j] > x ? 1 : 0;
+    }
+    if (r < n) sh.best[r] = x;
+  }
+  __syncthreads();
+}
+
+// sh.best[0, n): the n largest of the workgroup's packed keys v (0: none), descending.
+__device__ __forceinline__ void top_packed(const uint64_t (&v)[RE], int n, PickShared &sh) {
+  const int w = threadIdx.x >> 6;
+  uint64_t lm = 0;
+#pragma unroll
+  for (int i = 0; i < RE; ++i) lm = v[i] > lm ? v[i] : lm;
+  uint64_t thr = wave_kth_packed(lm, n);
+  thr = thr ? thr : 1ull;
+  uint32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < RE; ++i) {
+    const uint64_t bl = ballot64(v[i] >= thr);
+    if (bl) {
+      if (v[i] >= thr) sh.list[w][c + lanes_below(bl)] = v[i];
+      c += (uint32_t)__popcll(bl);
+    }
+  }
+  rank_lists(c, n, sh);
+}
+
+// A wave's n best tokens among its NV vectors from s0 on, one wave-wide maximum per token (read again each time): for a
+// wave whose elements at its threshold do not fit its list (many ties) or that has no threshold.
+template <int DT, bool AL>
+__device__ __noinline__ uint32_t top_by_rounds(const char *base, int s0, int V, int nv, int n, uint64_t *list) {
+  using L = RLay<DT>;
+  uint64_t prev = ~0ull;
+  uint32_t c = 0;
+  for (; c < (uint32_t)n; ++c) {
+    uint64_t m = 0;
+    for (int v = 0; v < nv; ++v) {
+      const int t0 = s0 + (v * RT + (int)threadIdx.x) * L::VEC;
+      float x[L::VEC];
+      load_vec<DT, AL>(base, t0, V, x);
+#pragma unroll
+      for (int e = 0; e < L::VEC; ++e) {
+        const uint64_t k = t0 + e < V ? pack(fkey(x[e]), (uint32_t)(t0 + e)) : 0ull;
+        m = k < prev && k > m ? k : m;
+      }
+    }
+    m = wave_max_u64(m);
+    if (!m) break;
+    if (lane_id() == 0) list[c] = m;
+    prev = m;
+  }
+  return c;
+}
+
+// sh.best[0, n): the packed keys of the n best tokens of the slice of NV vectors a thread from s0 on. A wave lists the
+// elements from the upper 16 key bits of its n-th largest lane maximum on: one maximum and one comparison per element.
+template <int DT, bool AL, int NV>
+__device__ __forceinline__ void top_tokens(const char *base, int s0, int V, int n, PickShared &sh) {
+  using L = RLay<DT>;
+  const int tid = threadIdx.x, w = tid >> 6;
+  float x[NV * L::VEC];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) load_vec<DT, AL>(base, s0 + (v * RT + tid) * L::VEC, V, &x[v * L::VEC]);
+  float lm = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NV * L::VEC; ++i) lm = fmaxf(lm, x[i]);
+  const uint32_t thr = wave_kth_largest_u16(fkey(lm) >> 16, n) << 16;
+  uint32_t c = TOPL + 1;
+  if (thr > KEY_NEGINF) {
+    const float xt = fkey_inv(thr);
+    c = 0;
+#pragma unroll
+    for (int i = 0; i < NV * L::VEC; ++i) {
+      const uint64_t bl = ballot64(x[i] >= xt);
+      if (bl) {
+        const uint32_t pos = c + lanes_below(bl);
+        if (x[i] >= xt && pos < (uint32_t)TOPL)
+          sh.list[w][pos] = pack(fkey(x[i]), (uint32_t)(s0 + (i / L::VEC * RT + tid) * L::VEC + i % L::VEC));
+        c += (uint32_t)__popcll(bl);
+      }
+    }
+  }
+  if (c > (uint32_t)TOPL) c = top_by_rounds<DT, AL>(base, s0, V, NV, n, sh.list[w]);
+  rank_lists(c, n, sh);
+}
+
+// Draw kd of a row whose slices are summed, by one wave.
+template <int DT>
+__device__ __forceinline__ void pick_draw(const PickArgs &a, int row, int kd, const char *base, double t,
+                                          const double *etab) {
+  using L = RLay<DT>;
+  const int lane = lane_id();
+  const size_t o = (size_t)row * a.ns;
+  const double *mx = a.max + o;
+  const Fx *ms = a.mass + o;
+  double M = -INFINITY;
+  for (int j = lane; j < a.ns; j += WAVE) M = fmax(M, ld_ag(&mx[j]));
+  M = lane63(wave_scan(M, (double)-INFINITY, [](double p, double q) { return fmax(p, q); }));
+  int tok = -1;
+  double lq = __builtin_nan("");
+  if (fabs(M) < INFINITY) {
+    auto weight = [&](int j) {
+      const double m = ld_ag(&mx[j]);
+      const Fx f{ld_ag(&ms[j].hi), ld_ag(&ms[j].lo)};
+      return m > -INFINITY ? fx_val(f) * exp_nonpos(m - M, etab) : 0.0;
+    };
+    double E = 0.0;
+    int last = -1;
+    for (int j0 = 0; j0 < a.ns; j0 += WAVE) {
+      const int j = j0 + lane;
+      const double x = j < a.ns ? weight(j) : 0.0;
+      if (x > 0.0) last = max(last, ld_ag(&a.last[o + j]));
+      E += wave_sum_f64(x);
+    }
+    last = (int)wave_max_u32((uint32_t)(last + 1)) - 1;
+    const double thr = uniform64(mix64(a.b.seed[row], SALT_DRAFT + (uint64_t)kd), a.b.at[row]) * E;
+    double before = 0.0;
+    const int sx = cross(a.ns, thr, before, weight);
+    tok = last;
+    if (sx >= 0) {
+      const double m = ld_ag(&mx[sx]), sc = exp_nonpos(m - M, etab);
+      const double ts = sc > 0.0 ? (thr - before) / sc : 0.0;  // the threshold in the slice's own masses
+      const Fx *sg = a.seg + (o + sx) * (RSEG / 2);
+      Fx f = lane < L::NSEG ? Fx{ld_ag(&sg[lane].hi), ld_ag(&sg[lane].lo)} : Fx{0, 0};
+      Fx inc{wave_incl_scan_u64(f.hi), wave_incl_scan_u64(f.lo)};
+      uint64_t hit = ballot64(lane < L::NSEG && fx_val(inc) >= ts);
+      tok = min(ld_ag(&a.last[o + sx]), last);  // (none: the slice's last token of positive mass)
+      if (hit) {
+        const int g = (int)__builtin_ctzll(hit);
+        const Fx b0{shfl_u64(inc.hi - f.hi, g), shfl_u64(inc.lo - f.lo, g)};
+        // the segment's masses again: lane l's VEC consecutive tokens
+        const int t0 = sx * RS + g * L::SEG + lane * L::VEC, V = (int)a.b.vocab;
+        Fx e[L::VEC], s{0, 0};
+#pragma unroll
+        for (int k = 0; k < L::VEC; ++k) {
+          const double z = logit_at<DT>(base, min(t0 + k, V - 1)) / t;
+          e[k] = t0 + k < V ? fx_of(exp_nonpos(z - m, etab)) : Fx{0, 0};
+          s = fx_add(s, e[k]);
+        }
+        Fx run = fx_add(b0, Fx{wave_incl_scan_u64(s.hi) - s.hi, wave_incl_scan_u64(s.lo) - s.lo});
+        int at = -1;
+#pragma unroll
+        for (int k = 0; k < L::VEC; ++k) {
+          run = fx_add(run, e[k]);
+          if (at < 0 && fx_val(run) >= ts) at = t0 + k;
+        }
+        hit = ballot64(at >= 0);
+        if (hit) tok = min(__shfl(at, (int)__builtin_ctzll(hit), WAVE), last);
+      }
+    }
+    if (tok >= 0) lq = (logit_at<DT>(base, tok) / t - M) - log(E);
+  }
+  if (lane == 0) {
+    a.b.out_tokens[(int64_t)row * a.b.out_ld + kd] = tok;
+    a.b.out_logq[(int64_t)row * a.b.out_ld + kd] = lq;
+  }
+}
+
+// The masses of one slice of a t > 0 row (slice index o over the rows' slices).
+template <int DT, bool AL>
+__device__ __forceinline__ void pick_masses(const PickArgs &a, const char *base, int s0, size_t o, double t,
+                                            PickShared &sh) {
+  using L = RLay<DT>;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6, V = (int)a.b.vocab;
+  float x[RE];
+#pragma unroll
+  for (int v = 0; v < L::NV; ++v) load_vec<DT, AL>(base, s0 + (v * RT + tid) * L::VEC, V, &x[v * L::VEC]);
+  float xm = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < RE; ++i) xm = fmaxf(xm, x[i]);
+  xm = wave_max_f32(xm);
+  if (lane == 0) sh.d.mx[w] = xm;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < RW; ++k) xm = fmaxf(xm, sh.d.mx[k]);
+  // (z = x / t is monotone in x and rounds once: the maximum of z is that of x divided)
+  const double m = t == 1.0 ? (double)xm : (double)xm / t;
+  int last = -1;
+  Fx tot{0, 0};
+#pragma unroll
+  for (int v = 0; v < L::NV; ++v) {
+    Fx f{0, 0};
+#pragma unroll
+    for (int e = 0; e < L::VEC; ++e) {
+      const double xd = (double)x[v * L::VEC + e], z = t == 1.0 ? xd : xd / t;
+      const double y = exp_nonpos(z - m, sh.etab);  // (0 for NaN and -inf)
+      f = fx_add(f, fx_of(y));
+      if (y > 0.0) last = s0 + (v * RT + tid) * L::VEC + e;
+    }
+    const Fx g{wave_sum_u64(f.hi), wave_sum_u64(f.lo)};
+    tot = fx_add(tot, g);
+    if (lane == 0) {  // segment v RW + w
+      Fx *sg = a.seg + o * (RSEG / 2) + v * RW + w;
+      st_ag(&sg->hi, g.hi);
+      st_ag(&sg->lo, g.lo);
+    }
+  }
+  last = (int)wave_max_u32((uint32_t)(last + 1)) - 1;
+  if (lane == 0) {
+    sh.d.shi[w] = tot.hi;
+    sh.d.slo[w] = tot.lo;
+    sh.d.last[w] = last;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    Fx f{0, 0};
+    int l = -1;
+    for (int k = 0; k < RW; ++k) {
+      f = fx_add(f, Fx{sh.d.shi[k], sh.d.slo[k]});
+      l = max(l, sh.d.last[k]);
+    }
+    st_ag(&a.max[o], m);
+    st_ag(&a.mass[o].hi, f.hi);
+    st_ag(&a.mass[o].lo, f.lo);
+    st_ag(&a.last[o], l);
+  }
+}
+
+// A workgroup takes SUB slices of its row: the slices of a t > 0 row one after the other, of a t == 0 row all at once.
+template <int DT, bool AL, int SUB>
+__global__ __launch_bounds__(RT) void pick_kernel(PickArgs a) {
+  using L = RLay<DT>;
+  __shared__ PickShared sh;
+  const int s = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, w = tid >> 6;
+  const int V = (int)a.b.vocab, ng = (int)gridDim.x;
+  const char *base = (const char *)a.b.x + (size_t)row * (size_t)a.b.ld * (DT == GSE_BF16 ? 2 : 4);
+  const double t = a.b.temperature[row];
+  const int n = min(max(a.b.n[row], 0), (int)min((int64_t)GSE_MAX_KIDS, a.b.out_ld));
+  if (n == 0) return;
+  if (tid < 64) sh.etab[tid] = EXP2_64[tid];  // (published by the first barrier)
+  const bool drawn = t > 0.0;
+  uint64_t *top = a.top + (size_t)row * a.ns * GSE_MAX_KIDS;
+  if (drawn) {
+    for (int j = s * SUB; j < min((s + 1) * SUB, a.ns); ++j) {
+      if (j > s * SUB) __syncthreads();  // (the LDS of the slice before)
+      pick_masses<DT, AL>(a, base, j * RS, (size_t)row * a.ns + j, t, sh);
+    }
+  } else {
+    top_tokens<DT, AL, SUB * L::NV>(base, s * SUB * RS, V, n, sh);
+    if (tid < n) st_ag(&top[s * GSE_MAX_KIDS + tid], sh.best[tid]);
+  }
+  store_wait();
+  __syncthreads();
+  if (tid == 0) sh.ticket = ticket_add(&a.tick[row]);
+  __syncthreads();
+  if (sh.ticket != (uint32_t)(ng - 1)) return;
+  // the row's last workgroup
+  if (tid == 0) a.tick[row] = 0;
+  if (drawn) {
+    for (int kd = w; kd < n; kd += RW) pick_draw<DT>(a, row, kd, base, t, sh.etab);
+    return;
+  }
+  const int N = ng * n;  // entry i: the (i % n)-th best of workgroup i / n
+  for (int i0 = 0; i0 < N; i0 += RT * (RE - 1)) {  // (the last element of each thread carries the best so far)
+    uint64_t v[RE];
+#pragma unroll
+    for (int k = 0; k < RE; ++k) {
+      const int i = i0 + k * RT + tid;
+      v[k] = 0ull;
+      if (k == RE - 1) v[k] = i0 > 0 && tid < n ? sh.best[tid] : 0ull;
+      else if (i0 + k * RT < N && i < N) v[k] = ld_ag(&top[(size_t)(i / n) * GSE_MAX_KIDS + i % n]);
+    }
+    __syncthreads();
+    top_packed(v, n, sh);
+  }
+  if (tid < n) {
+    const uint64_t pk = sh.best[tid];
+    const int id = pk ? (int)pk_id(pk) : -1;
+    a.b.out_tokens[(int64_t)row * a.b.out_ld + tid] = id;
+    a.b.out_logq[(int64_t)row * a.b.out_ld + tid] = id >= 0 ? logit_at<DT>(base, id) : __builtin_nan("");
+  }
+}
+
 // The slicing of rows of V tokens, and the rows that one launch takes (at least 1) of the workspace's R rows of S slices.
 RowSlices slices_of(const RowsWs &w, int V, int *rows) {
   const int64_t cap = (int64_t)w.rows * w.slices;
@@ -431,6 +819,39 @@ hipError_t launch_mss(const RowsWs &w, const gse_mss_batch &b, hipStream_t s) {
     if (b.max_kids > 1) hipLaunchKernelGGL(mss_kernel<2>, grid, block, 0, s, a);
     if (b.max_kids > 2) hipLaunchKernelGGL(mss_kernel<3>, grid, block, 0, s, a);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_pick(const RowsWs &w, const gse_pick_batch &b, hipStream_t s) {
+  PickArgs a;
+  a.b = b;
+  a.ns = ((int)b.vocab + RS - 1) / RS;  // (at most w.slices, and at most w.rows rows: the caller's checks)
+  a.max = w.sum;
+  a.mass = w.mass;
+  a.seg = (Fx *)w.seg;
+  a.last = w.last;
+  a.top = w.top;
+  a.tick = w.tick;
+  // whole 16-byte vectors when every row starts on a 16-byte boundary
+  const bool al = ((((uintptr_t)b.x) | ((uintptr_t)b.ld * (b.dtype == GSE_BF16 ? 2u : 4u))) & 15u) == 0;
+  // One slice per workgroup while the call's slices fit the device at once (four workgroups per CU), else four: every
+  // workgroup ends with the same chain (list, ranks, store, ticket), so past one round the longer ones win.
+  const bool wide = (int64_t)a.ns * b.rows > w.round;
+  auto go = [&](auto dt, auto aligned, auto sub) {
+    constexpr int SUB = decltype(sub)::value;
+    hipLaunchKernelGGL((pick_kernel<decltype(dt)::value, decltype(aligned)::value, SUB>),
+                       dim3((a.ns + SUB - 1) / SUB, b.rows), dim3(RT), 0, s, a);
+  };
+  auto by_sub = [&](auto dt, auto aligned) {
+    if (wide) go(dt, aligned, std::integral_constant<int, 4>{});
+    else go(dt, aligned, std::integral_constant<int, 1>{});
+  };
+  auto by_al = [&](auto dt) {
+    if (al) by_sub(dt, std::true_type{});
+    else by_sub(dt, std::false_type{});
+  };
+  if (b.dtype == GSE_BF16) by_al(std::integral_constant<int, (int)GSE_BF16>{});
+  else by_al(std::integral_constant<int, (int)GSE_F32>{});
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 // Speculative decoding on the device: the acceptance walk of a verify round (goethe_engine/engine.py:262-298 with
-// spec.py:88-103 mss at strict nodes) and the drafter's child selection (spec.py:151-159 TreeDrafter._pick).
+// spec.py:88-103 mss at strict nodes).
 //
 // Verify. A node's outcome does not depend on the path that reaches it: its uniform index is nout0 + depth (one token
 // is committed per level, engine.py:272,282) and its target row, mask and history are fixed by the path to it. So every
@@ -17,10 +17,6 @@
 //      holding it (engine.py:284-285); a token -1 ends the walk as an error (engine.py:286-288).
 // Every slice of a node computes the same values from the same partials, read in slice order, so the decisions are
 // deterministic and identical in every workgroup.
-//
-// Pick. t == 0: the n largest tokens in stable descending order (ties to the lowest id), per slice then merged by the
-// row's last slice. t > 0: the maximum of z = x / t, the exact mass E = sum(exp(z - M)) in fixed point per slice, then
-// one workgroup per draw k finds the first index whose inclusive prefix reaches uniform(mix(seed, 2^42 + k), at) * E.
 #include <type_traits>
 
 #include "gse_rowctx.h"
@@ -31,9 +27,8 @@ namespace {
 
 constexpr int TT = 256;          // threads per slice workgroup
 constexpr int TS = CH;           // tokens per slice
-constexpr int TK = TS / TT;      // tokens per thread (strided: token s0 + k * TT + tid)
 constexpr int TSEG = TS / WAVE;  // 64-token segments of a slice
-constexpr uint64_t SALT_ACC = 1ull << 40, SALT_RES = 1ull << 41, SALT_DRAFT = 1ull << 42;
+constexpr uint64_t SALT_ACC = 1ull << 40, SALT_RES = 1ull << 41;
 
 // ---- fixed-point helpers -------------------------------------------------------------------------------------------
 
@@ -700,12 +695,6 @@ __device__ __forceinline__ int slice_find(int s0, int s1, Fx before, double thr,
 
 // ---- verify: stats --------------------------------------------------------------------------------------------------
 
-__device__ __forceinline__ bool node_live(const TreeArgs &a, int u, const gse_row &P) {
-  if (!(P.flags & GSE_ROW_MSS)) return false;
-  const uint32_t f = a.s.info[u].flags;
-  return (f & R_DONE) && !(f & (R_SPECIAL | R_BAD | R_GREEDY));
-}
-
 __device__ __forceinline__ Tgt tgt_of(const TreeArgs &a, int u, const gse_row &P) {
   Tgt g;
   g.c = make_ctx(a.s, u, P);
@@ -727,7 +716,7 @@ __global__ __launch_bounds__(TT) void tstats_kernel(TreeArgs a) {
   if (y < a.nodes) {
     const int u = y;
     const gse_row P = a.s.params[u];
-    const uint32_t inf = a.s.info[u].flags;  // (node_live in place: one round of loads, as in tkid0_kernel)
+    const uint32_t inf = a.s.info[u].flags;  // (one round of loads, as in tkid0_kernel)
     const Tgt g = tgt_of(a, u, P);
     if (!(P.flags & GSE_ROW_MSS) || !(inf & R_DONE) || (inf & (R_SPECIAL | R_BAD | R_GREEDY))) return;
     load_etab(sh);
@@ -969,7 +958,7 @@ __global__ __launch_bounds__(TT) void tkid0_kernel(TreeArgs a) {
   const gse_row P = a.s.params[u];
   TreeNode &nd = a.st[u];
   // the row's flags, its state and its target fields in one round of loads (a load behind a branch waits for the
-  // branch's own): node_live in place
+  // branch's own)
   const uint32_t inf = a.s.info[u].flags;
   const int next = (int)nd.next;
   const Tgt g = tgt_of(a, u, P);
@@ -998,7 +987,7 @@ __device__ __forceinline__ void tpass_item(const TreeArgs &a, int r, int u, int 
   const int tid = threadIdx.x;
   const gse_row P = a.s.params[u];
   TreeNode &nd = a.st[u];
-  const uint32_t inf = a.s.info[u].flags;  // (node_live in place: one round of loads, as in tkid0_kernel)
+  const uint32_t inf = a.s.info[u].flags;  // (one round of loads, as in tkid0_kernel)
   const int next = (int)nd.next;
   const Tgt g = tgt_of(a, u, P);
   if (!(P.flags & GSE_ROW_MSS) || !(inf & R_DONE) || (inf & (R_SPECIAL | R_BAD | R_GREEDY)) || next != r) return;
@@ -1180,7 +1169,7 @@ __device__ __forceinline__ WalkNode walk_node(const TreeArgs &a, int u, int end)
   return w;
 }
 
-// node_live from the loaded flags
+// a node that takes dist + mss and whose row has a distribution, from the loaded flags
 __device__ __forceinline__ bool walk_live(const WalkNode &w) {
   return (w.pf & GSE_ROW_MSS) && (w.inf & R_DONE) && !(w.inf & (R_SPECIAL | R_BAD | R_GREEDY));
 }
@@ -1278,165 +1267,6 @@ __global__ __launch_bounds__(64) void walk_kernel(TreeArgs a) {
   if (a.out.status) a.out.status[q] = status;
 }
 
-// ---- pick (spec.py:151-159) -----------------------------------------------------------------------------------------
-
-struct PickArgs {
-  gse_pick_batch b;
-  int nsl;
-  double *pmax;     // [rows][nsl]
-  Fx *ppart;        // [rows][nsl]
-  int32_t *plast;   // [rows][nsl]
-  uint64_t *ptop;   // [rows][nsl][4 * GSE_MAX_KIDS] packed (key, id) top candidates per wave
-  uint32_t *tick;   // [rows]
-};
-
-__device__ __forceinline__ float pick_x(const PickArgs &a, int row, int i) {
-  const char *base = (const char *)a.b.x + (size_t)row * (size_t)a.b.ld * (a.b.dtype == GSE_BF16 ? 2 : 4);
-  return a.b.dtype == GSE_BF16 ? bf16_to_f32(((const uint16_t *)base)[i]) : ((const float *)base)[i];
-}
-
-// t > 0: the maximum of z = x / t per slice. t == 0: the top-n packed (key(x), id) of each wave of the slice, then the
-// row's last slice merges them (bitonic sort in LDS) and writes the n best.
-__global__ __launch_bounds__(TT) void pick1_kernel(PickArgs a) {
-  __shared__ double red[8];
-  __shared__ uint64_t cand[TT / WAVE * GSE_MAX_KIDS * 32];
-  __shared__ uint32_t ticket;
-  const int s = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-  const int V = (int)a.b.vocab, s0 = s * TS, s1 = min(V, s0 + TS);
-  const double t = a.b.temperature[row];
-  const int n = min(max(a.b.n[row], 0), (int)min((int64_t)GSE_MAX_KIDS, a.b.out_ld));
-  if (t > 0.0) {
-    double m = -INFINITY;
-    for (int i = s0 + tid; i < s1; i += TT) m = fmax(m, (double)pick_x(a, row, i) / t);
-    m = block_max_f64(m, red);
-    if (tid == 0) a.pmax[(size_t)row * a.nsl + s] = m;
-    return;
-  }
-  if (n == 0) return;
-  uint64_t v[TK];
-  for (int k = 0; k < TK; ++k) {
-    const int i = s0 + k * TT + tid;
-    v[k] = i < s1 ? pack(fkey(pick_x(a, row, i)), (uint32_t)i) : 0ull;
-  }
-  // n rounds of the wave maximum, the winner removed
-  uint64_t *wc = a.ptop + ((size_t)row * a.nsl + s) * (TT / WAVE) * GSE_MAX_KIDS + (tid >> 6) * GSE_MAX_KIDS;
-  for (int r = 0; r < n; ++r) {
-    uint64_t lm = 0;
-    for (int k = 0; k < TK; ++k) lm = v[k] > lm ? v[k] : lm;
-    const uint64_t wm = wave_max_u64(lm);
-    for (int k = 0; k < TK; ++k)
-      if (v[k] == wm) v[k] = 0ull;
-    if (lane_id() == 0) st_ag(&wc[r], wm);
-  }
-  store_wait();
-  __syncthreads();
-  if (tid == 0) ticket = ticket_add(&a.tick[row]);
-  __syncthreads();
-  if (ticket != (uint32_t)(a.nsl - 1)) return;
-  // merge the nsl * 4 lists of n in rounds of the LDS buffer, carrying the best n
-  const int tot = a.nsl * (TT / WAVE) * GSE_MAX_KIDS;
-  const uint64_t *all = a.ptop + (size_t)row * a.nsl * (TT / WAVE) * GSE_MAX_KIDS;
-  uint64_t best[GSE_MAX_KIDS];
-  for (int r = 0; r < GSE_MAX_KIDS; ++r) best[r] = 0ull;
-  const int cap = TT / WAVE * GSE_MAX_KIDS * 32;
-  for (int b0 = 0; b0 < tot; b0 += cap - GSE_MAX_KIDS) {
-    // the buffer: the best so far, then the next entries
-    const int nb = min(cap, GSE_MAX_KIDS + (tot - b0));
-    const int np = pow2_ceil(nb);
-    for (int i = tid; i < np; i += TT) {
-      uint64_t x = 0ull;
-      const int e = b0 + i - GSE_MAX_KIDS;  // entry of the lists: [slice][wave][GSE_MAX_KIDS], the first n filled
-      if (i < GSE_MAX_KIDS) x = best[i];
-      else if (i < nb && e % GSE_MAX_KIDS < n) x = ld_ag(&all[e]);
-      cand[i] = x;
-    }
-    __syncthreads();
-    block_sort_desc_u64(cand, np);
-    for (int r = 0; r < GSE_MAX_KIDS; ++r) best[r] = r < n ? cand[r] : 0ull;
-    __syncthreads();
-  }
-  if (tid < n) {
-    const uint64_t pk = best[tid];
-    const int id = pk ? (int)pk_id(pk) : -1;
-    a.b.out_tokens[(int64_t)row * a.b.out_ld + tid] = id;
-    a.b.out_logq[(int64_t)row * a.b.out_ld + tid] = id >= 0 ? (double)pick_x(a, row, id) : __builtin_nan("");
-  }
-  if (tid == 0) a.tick[row] = 0;
-}
-
-// t > 0: exact partial masses exp(z - M) per slice.
-__global__ __launch_bounds__(TT) void pick2_kernel(PickArgs a) {
-  __shared__ uint64_t red[16];
-  __shared__ int redi[8];
-  const int s = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-  const double t = a.b.temperature[row];
-  if (!(t > 0.0) || a.b.n[row] <= 0) return;
-  const int V = (int)a.b.vocab, s0 = s * TS, s1 = min(V, s0 + TS);
-  double M = -INFINITY;
-  for (int j = lane_id(); j < a.nsl; j += WAVE) M = fmax(M, a.pmax[(size_t)row * a.nsl + j]);
-  M = wave_max_f64(M);
-  Fx f = fx_zero();
-  int last = -1;
-  for (int k = 0; k < TK; ++k) {
-    const int i = s0 + k * TT + tid;
-    if (i >= s1) break;
-    const double e = exp((double)pick_x(a, row, i) / t - M);
-    f = fx_add(f, fx_of(e));
-    if (e > 0.0) last = i;
-  }
-  f = block_fx_sum(f, red);
-  last = block_max_i32(last, redi);
-  if (tid == 0) {
-    a.ppart[(size_t)row * a.nsl + s] = f;
-    a.plast[(size_t)row * a.nsl + s] = last;
-  }
-}
-
-// t > 0: one workgroup per (row, draw k): draw(q, uniform(mix(seed, SALT_DRAFT + k), at)) in vocabulary order.
-__global__ __launch_bounds__(TT) void pick3_kernel(PickArgs a) {
-  __shared__ TreeShared sh;
-  const int row = blockIdx.y, kd = blockIdx.x, tid = threadIdx.x;
-  const double t = a.b.temperature[row];
-  const int n = min(max(a.b.n[row], 0), (int)min((int64_t)GSE_MAX_KIDS, a.b.out_ld));
-  if (!(t > 0.0) || kd >= n) return;
-  const int V = (int)a.b.vocab;
-  // (every wave reads the row's partials itself, a slice per lane)
-  const double *pm = a.pmax + (size_t)row * a.nsl;
-  const Fx *pp = a.ppart + (size_t)row * a.nsl;
-  const int32_t *pl = a.plast + (size_t)row * a.nsl;
-  double M = -INFINITY;
-  int lastl = -1;
-  for (int j = lane_id(); j < a.nsl; j += WAVE) {
-    M = fmax(M, pm[j]);
-    lastl = max(lastl, pl[j]);
-  }
-  M = wave_max_f64(M);
-  const int last = (int)wave_max_u32((uint32_t)(lastl + 1)) - 1;
-  auto part = [&](int j) { return pp[j]; };
-  const Fx tot = wave_fx_total(a.nsl, part);
-  int tok = -1;
-  double lq = __builtin_nan("");
-  if (last >= 0) {
-    const double E = fx_val(tot);
-    const double thr = uniform64(mix64(a.b.seed[row], SALT_DRAFT + (uint64_t)kd), a.b.at[row]) * E;
-    Fx before;
-    const int sx = wave_fx_cross(a.nsl, thr, part, before);
-    const int s0 = sx * TS, s1 = min(V, s0 + TS);
-    const int j = slice_find(s0, s1, before, thr, [&](int i) { return pick_x(a, row, i); },
-                             [&](int, float x) { return exp((double)x / t - M); }, sh);
-    tok = j < 0 ? last : min(j, last);
-    lq = ((double)pick_x(a, row, tok) / t - M) - log(E);
-  }
-  if (tid == 0) {
-    a.b.out_tokens[(int64_t)row * a.b.out_ld + kd] = tok;
-    a.b.out_logq[(int64_t)row * a.b.out_ld + kd] = lq;
-  }
-}
-
-}  // namespace
-
-namespace {
-
 TreeArgs tree_args(const TreeLaunch &L) {
   TreeArgs a;
   a.s = L.s;
@@ -1497,22 +1327,6 @@ hipError_t launch_tree(const TreeLaunch &L, hipStream_t s) {
   };
   by_instance(L, go);
   hipLaunchKernelGGL(walk_kernel, dim3((max(a.requests, a.nodes) + 63) / 64), dim3(64), 0, s, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_pick(const PickLaunch &L, hipStream_t s) {
-  PickArgs a;
-  a.b = L.b;
-  a.nsl = ((int)L.b.vocab + TS - 1) / TS;
-  a.pmax = L.pmax;
-  a.ppart = L.ppart;
-  a.plast = L.plast;
-  a.ptop = L.ptop;
-  a.tick = L.tick;
-  const int nmax = (int)min((int64_t)GSE_MAX_KIDS, L.b.out_ld);
-  hipLaunchKernelGGL(pick1_kernel, dim3(a.nsl, L.b.rows), dim3(TT), 0, s, a);
-  hipLaunchKernelGGL(pick2_kernel, dim3(a.nsl, L.b.rows), dim3(TT), 0, s, a);
-  hipLaunchKernelGGL(pick3_kernel, dim3(nmax, L.b.rows), dim3(TT), 0, s, a);
   return hipGetLastError();
 }
 

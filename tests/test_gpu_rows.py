@@ -1,4 +1,4 @@
-"""GPU parity of the row passes (draw, mss) at the edges of their slices and segments, against the oracle: tokens and
+"""GPU parity of the row passes (draw, mss, pick) at the edges of their slices and segments, against the oracle: tokens and
 accepted kids are compared exactly (a draw within rounding of a prefix boundary has a probability of about 1e-13)."""
 import ctypes as C
 
@@ -108,3 +108,72 @@ def test_rows_past_the_handles_size(ge, gpu):
     assert ot.cpu().tolist() == [t for t, _ in want]
     assert ok.cpu().tolist() == [-1 if r is None else r for _, r in want]
     h.close()
+
+
+def _pick_rows(v, rng):
+    """Rows with ties everywhere (one value; two values), with the best tokens side by side, with -inf in most places,
+    with a single finite token, and plain ones."""
+    x = rng.normal(0, 3, size=(7, v)).astype(np.float32)
+    x[1] = 0.25
+    x[2] = (rng.random(v) < 0.5).astype(np.float32)
+    x[3, v // 2:v // 2 + 20] += 30.0
+    x[4, rng.random(v) < 0.99] = -np.inf
+    x[4, -1] = 1.0
+    x[5] = -np.inf
+    x[5, v // 3] = -2.0
+    return x
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("v", [1, 5, 64, 255, 4095, 4096, 4097, 50257, 262147])
+def test_pick_sizes(ge, gpu, v, shift, dtype):
+    """n best and n draws (n to 16) over whole and ragged slices, rows on and off a 16-byte boundary, t == 0 and t > 0
+    rows in one call."""
+    rng = np.random.default_rng(v + shift)
+    x = torch.from_numpy(_pick_rows(v, rng))
+    x = x.bfloat16() if dtype == "bf16" else x
+    x32 = x.float().numpy()
+    rows = len(x)
+    buf = torch.zeros((rows, v + 3), dtype=x.dtype)
+    buf[:, shift:shift + v] = x
+    xd = buf.to(gpu)[:, shift:shift + v] if v > 1 else x.to(gpu)
+    for t in ([0.0] * rows, [0.7] * rows, [0.0, 1.0, 1.0, 0.0, 2.5, 0.5, 1.0]):
+        n = [min(v, k) for k in (16, 1, 7, 16, 3, 1, 4)]
+        if t[4] == 0.0:  # (as many as there are tokens above -inf: the oracle then has no tie to break past them)
+            n[4] = min(3, int((x32[4] > -np.inf).sum()))
+        seeds, ats = [1000 + r for r in range(rows)], [3 * r for r in range(rows)]
+        toks, vals = ge.spec.pick_batch(xd, n, t, seeds, ats)
+        toks, vals = toks.cpu().numpy(), vals.cpu().numpy()
+        for r in range(rows):
+            want = spo.pick(x32[r], n[r], t[r], seeds[r], ats[r])
+            assert list(toks[r, :n[r]]) == [w[0] for w in want], (v, t[r], r)
+            np.testing.assert_allclose(vals[r, :n[r]], [w[2] for w in want], rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_pick_more_slices_than_the_device_holds(ge, gpu, dtype):
+    """300 rows of five slices (the last one of five tokens): the workgroups take four slices each, ties and all, and the
+    draws' values are those of the same rows alone."""
+    rng = np.random.default_rng(17)
+    v, rows = 4 * 4096 + 5, 301
+    x = torch.from_numpy(np.concatenate([_pick_rows(v, rng) for _ in range(43)]))
+    x = x.bfloat16() if dtype == "bf16" else x
+    x32, xd = x.float().numpy(), x.to(gpu)
+    n = [int(k) for k in rng.integers(1, 17, size=rows)]
+    t = [float(k) for k in rng.choice([0.0, 0.0, 0.6, 1.0], size=rows)]
+    seeds, ats = list(range(rows)), [7] * rows
+    for r in range(rows):
+        if t[r] == 0.0 and r % 7 in (4, 5):
+            n[r] = min(n[r], int((x32[r] > -np.inf).sum()))
+    toks, vals = ge.spec.pick_batch(xd, n, t, seeds, ats)
+    toks, vals = toks.cpu().numpy(), vals.cpu().numpy()
+    for r in range(rows):
+        want = spo.pick(x32[r], n[r], t[r], seeds[r], ats[r])
+        assert list(toks[r, :n[r]]) == [w[0] for w in want], (t[r], r)
+        np.testing.assert_allclose(vals[r, :n[r]], [w[2] for w in want], rtol=1e-12, atol=1e-12)
+    some = list(range(0, rows, 20))
+    t1, v1 = ge.spec.pick_batch(xd[some], [n[r] for r in some], [t[r] for r in some], some, [7] * len(some))
+    t1, v1 = t1.cpu().numpy(), v1.cpu().numpy()
+    for i, r in enumerate(some):
+        assert list(t1[i, :n[r]]) == list(toks[r, :n[r]]) and np.array_equal(v1[i, :n[r]], vals[r, :n[r]])
