@@ -544,7 +544,7 @@ GSE_API int gse_qprob(gse_handle *h, const gse_qrows *qrows, uint32_t vocab, dou
   if (vocab == 0 || q.ld < (int64_t)vocab || out_ld < (int64_t)vocab)
     return fail(h, GSE_E_ARG, "vocab 0, q ld < vocab or out_ld < vocab");
   DeviceGuard g(h->device);
-  hipError_t e = gse::launch_qprob(q, (int)vocab, out, out_ld, (hipStream_t)stream);
+  hipError_t e = gse::launch_qprob(rows_ws(h), q, (int)vocab, out, out_ld, (hipStream_t)stream);
   return e == hipSuccess ? GSE_OK : hip_fail(h, e, "qprob launch");
 }
 

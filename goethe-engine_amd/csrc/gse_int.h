@@ -269,15 +269,15 @@ hipError_t launch_main(const ScanArgs &a, hipStream_t s);
 hipError_t launch_deep(const ScanArgs &a, hipStream_t s);
 hipError_t launch_exact(const ScanArgs &a, hipStream_t s);
 hipError_t launch_dist_write(const ScanArgs &a, double *probs, int64_t probs_ld, hipStream_t s);
-// Row passes (gse_rows.hip): draw() and mss() over fp64 rows, the drafter's picks.
+// Row passes (gse_rows.hip): draw() and mss() over fp64 rows, the drafter's picks and its softmax rows.
 hipError_t launch_draw(const RowsWs &w, const double *q, int64_t ld, int rows, int V, const double *u, int32_t *out,
                        hipStream_t s);
 hipError_t launch_mss(const RowsWs &w, const gse_mss_batch &b, hipStream_t s);
 // The verify round after the selection pass (the statistics of the q rows given as drafter logits included).
 hipError_t launch_tree(const TreeLaunch &L, hipStream_t s);
 hipError_t launch_pick(const RowsWs &w, const gse_pick_batch &b, hipStream_t s);
+hipError_t launch_qprob(const RowsWs &w, const gse_qrows &q, int V, double *out, int64_t ld, hipStream_t s);
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
-hipError_t launch_qprob(const gse_qrows &q, int V, double *out, int64_t ld, hipStream_t s);
 hipError_t launch_pack(const uint8_t *bools, int64_t bld, int rows, int V, int32_t *words, int64_t wld, hipStream_t s);
 
 }  // namespace gse

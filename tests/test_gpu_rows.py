@@ -177,3 +177,40 @@ def test_pick_more_slices_than_the_device_holds(ge, gpu, dtype):
     t1, v1 = t1.cpu().numpy(), v1.cpu().numpy()
     for i, r in enumerate(some):
         assert list(t1[i, :n[r]]) == list(toks[r, :n[r]]) and np.array_equal(v1[i, :n[r]], vals[r, :n[r]])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("v", [1, 4095, 4097, 50257])
+def test_qprob_sizes(ge, gpu, v, dtype):
+    """Softmax rows over whole and ragged slices, on and off a 16-byte boundary, with -inf, masses far below the row's
+    maximum, and the rows that are NaN everywhere (a NaN, a +inf, nothing above -inf); and the same through a handle whose
+    few slices widen. q = exp(z - M) / E: each of z, the exponential, the sum and the quotient rounds within an ulp or two,
+    and z's rounding (|z| 2^-53) is an error of the exponent, so 1e-13 covers |z| up to a few hundred."""
+    rng = np.random.default_rng(v)
+    x = torch.from_numpy(np.concatenate([_pick_rows(v, rng), np.full((3, v), 1.5, np.float32)]))
+    x[0, 0] = -700.0
+    x[7, v // 2] = np.nan
+    x[8, v - 1] = np.inf
+    x[9] = -np.inf
+    x = x.bfloat16() if dtype == "bf16" else x
+    x64 = x.double().numpy()
+    t = [1.0, 0.5, 1.7, 2.0, 0.9, 1.0, 0.3, 1.0, 0.7, 1.0]
+    buf = torch.zeros((len(x), v + 1), dtype=x.dtype)
+    buf[:, 1:] = x
+    outs = [ge.spec.qprob(x.to(gpu), t), ge.spec.qprob(buf.to(gpu)[:, 1:] if v > 1 else x.to(gpu), t)]
+    lib = ge._lib
+    h = lib.Handle(gpu.index, 1, 64)
+    xd, td = x.to(gpu), torch.tensor(t, dtype=torch.float64, device=gpu)
+    out = torch.full((len(x), v), -1.0, dtype=torch.float64, device=gpu)
+    q = lib.QRows()
+    q.size, q.kind = C.sizeof(lib.QRows), lib.Q_LOGITS_BF16 if dtype == "bf16" else lib.Q_LOGITS_F32
+    q.rows, q.q, q.ld, q.temperature = len(x), xd.data_ptr(), v, td.data_ptr()
+    h.call("gse_qprob", C.byref(q), v, out.data_ptr(), v, lib.stream_of(gpu.index))
+    outs.append(out)
+    for got in (o.cpu().numpy() for o in outs):
+        assert np.isnan(got[7:]).all()
+        for r in range(7):
+            z = x64[r] / t[r]
+            e = np.exp(z - z.max())
+            np.testing.assert_allclose(got[r], e / e.sum(), rtol=1e-13, atol=1e-300)
+    h.close()
