@@ -7,7 +7,7 @@
 //
 //   count:  each slice recomputes z exactly as the main pass does and adds a 512-bin histogram of
 //           d = z_max - z: counts and exact fixed-point masses (fp64 exp, whole multiples of 2^-40 and 2^-64; bins
-//           1/32 wide, the last one open-ended). d is monotone in z, so the bins follow the stable order and ties share
+//           1/32 wide, wider past d = 12, the last one open). d is monotone in z, so the bins follow the stable order and ties share
 //           a bin. The row's last slice plans: the bins that hold the last kept element (top-p, top-k and min-p cuts)
 //           and the bins that may hold the draw, whether they hold at most DCAP elements, and the exact masses of the
 //           regions before and between them; then it publishes the plan's status.
@@ -29,7 +29,11 @@ namespace {
 
 using namespace strm;
 
-constexpr float BSC = 32.0f;    // bins per unit of d
+// Histogram bins of d = z_max - z: 1/32 wide to d = 12 (bin 384), 1/8 wide to d = 20 (bin 448), then 1/2 wide; the last one
+// (from d = 51.5) is open. Most rows' cuts lie in the fine bins; the wide ones spread the tail of a row whose logits range
+// far (a keep set that ends past d = 16: top-p at or near 1), whose tens of thousands of elements in one open bin no window
+// list holds (such a row took the exact path: 460 us at V = 50257).
+constexpr float BSC = 32.0f;    // fine bins per unit of d
 constexpr int BPT = DNB / MT;   // planner: bins per thread (contiguous)
 constexpr int WLC = 1024;       // window elements a slice gathers in LDS before one global reservation (the histogram's space)
 static_assert(BPT * MT == DNB, "");
@@ -54,10 +58,12 @@ struct DeepShared {
   uint64_t pub[6];
 };
 
-// Bin of z (z > -inf, z <= M): monotone non-increasing in z.
-__device__ __forceinline__ uint32_t dbin(float z, float M) {
-  return (uint32_t)fminf((M - z) * BSC, (float)(DNB - 1));
+// The fractional bin of a distance t = d BSC: the least of the three widths' lines, monotone in t.
+__device__ __forceinline__ float bin_of(float t) {
+  return fminf(fminf(t, fmaf(t, 0.25f, 288.0f)), fminf(fmaf(t, 0.0625f, 408.0f), (float)(DNB - 1)));
 }
+// Bin of z (z > -inf, z <= M): monotone non-increasing in z.
+__device__ __forceinline__ uint32_t dbin(float z, float M) { return (uint32_t)bin_of((M - z) * BSC); }
 
 __device__ __forceinline__ void atomic_add_ag(uint64_t *p, uint64_t v) {
   (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -209,12 +215,14 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
     mh[j] = ld_ag(&gh[DNB + tid * BPT + j]);
     mo[j] = ld_ag(&gh[2 * DNB + tid * BPT + j]);
   }
-  // min-p keeps exp(z - M) >= min_p, i.e. d <= -ln(min_p): bins below bm - 1 are all kept, bins above bm + 1 all cut
+  // min-p keeps exp(z - M) >= min_p, i.e. d <= -ln(min_p): bins below bmlo are all kept, bins above bmhi all cut (an
+  // element's bin and -ln(min_p) are each off by less than 1e-4 bins: fp32 roundings of d BSC <= 1648)
   const bool mp = min_p > 0.0;
-  uint32_t bm = 0;
+  uint32_t bmlo = 0, bmhi = 0;
   if (mp) {
-    const double dm = -log(min_p) * (double)BSC;
-    bm = dm >= (double)(DNB - 1) ? (uint32_t)(DNB - 1) : (uint32_t)dm;
+    const float t = (float)fmin(-log(min_p) * (double)BSC, 1e6);
+    bmlo = (uint32_t)fmaxf(bin_of(t) - 0.01f, 0.0f);
+    bmhi = min((uint32_t)(bin_of(t) + 0.01f), (uint32_t)(DNB - 1));
   }
   // inclusive prefixes through each bin: counts, exact masses (2^-40 and 2^-64 parts) and their fp64 values
   uint64_t cl = 0, hl = 0, ol = 0;
@@ -268,8 +276,8 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
   // the windows of the cuts:
   //   b0, b1: first bins with inclusive mass >= tS - delta, >= tS + delta (top-p: the bin of the last kept element)
   //   b2:     first bin with inclusive count >= K (top-k: the bin of rank K - 1)
-  //   b5 - 1: last non-empty bin below bm - 1 (min-p: holds a kept element, so the last kept one is at or after it)
-  //   b6:     first non-empty bin above bm + 1 (min-p: holds a cut element)
+  //   b5 - 1: last non-empty bin below bmlo (min-p: all kept, so the last element it keeps is there or after it)
+  //   b6:     first non-empty bin above bmhi (min-p: all cut)
   {
     uint32_t b0 = DNB - 1, b1 = DNB - 1, b2 = DNB - 1, b5 = 0, b6 = DNB - 1;
 #pragma unroll
@@ -278,13 +286,13 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
       if (pm[j] >= tS - delta) b0 = b;
       if (pm[j] >= tS + delta) b1 = b;
       if (pc[j] >= K) b2 = b;
-      if (mp && c[j] && b > bm + 1) b6 = b;
+      if (mp && c[j] && b > bmhi) b6 = b;
     }
     if (mp) {
 #pragma unroll
       for (int j = 0; j < BPT; ++j) {
         const uint32_t b = tid * BPT + j;
-        if (c[j] && b + 1 < bm) b5 = b + 1;
+        if (c[j] && b < bmlo) b5 = b + 1;
       }
     }
     b0 = wave_min_u32(b0);
@@ -307,17 +315,25 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
     w1hi = min(w1hi, sh.q[PQ_B2]);
   }
   if (mp) {
+    // The first cut element comes at or before each cut's own: in the window that ends where the earlier cut is sure. A
+    // window that ends before min-p's first sure cut (hi) ends in a bin by which top-p or top-k has cut. (A window from
+    // the one cut to the other held more elements than the list in flat rows, and 40 % of the C3 batches of other seeds
+    // had such a row on the exact path: 0.9 - 3.8 ms a call where 115 us is usual.)
     const uint32_t b5 = sh.q[PQ_B5], lo = b5 ? b5 - 1u : 0u, hi = sh.q[PQ_B6];
     w1lo = min(w1lo, lo);
-    // when min-p may bind, the window reaches its first cut element (the finish cannot test min-p unlisted)
-    w1hi = lo <= w1hi ? max(w1hi, min(hi, (uint32_t)(DNB - 1))) : min(w1hi, hi);
+    w1hi = min(w1hi, hi);
   }
+  // A sampled row that keeps everything (c_last = S) needs no cut window. (The exact prefix test of sampling.py:80 with
+  // top_p = 1 cuts elements whose whole remaining mass is below 2^-53 S: c_last is S within that rounding.)
+  const bool all = mode == MODE_SAMPLE && top_p >= 1.0 && K >= ctot && !mp;
+  if (all) w1lo = w1hi = DNB - 1;
   auto at = [&](const auto *t, int b) { return b < 0 ? decltype(t[0])(0) : t[b]; };
   // masses before w1lo and through w1hi, then the windows of the draw
   uint32_t w2lo = w1lo, w2hi = w1hi;
   if (mode == MODE_SAMPLE) {
-    const double qd0 = fx_val(Fx{at(sh.ph, (int)w1lo - 1), at(sh.po, (int)w1lo - 1)});  // (pm of those bins)
-    const double qd1 = fx_val(Fx{at(sh.ph, (int)w1hi), at(sh.po, (int)w1hi)});
+    // c_last lies between the masses through the bins at the cut window's edges (pm of those bins)
+    const double qd0 = all ? S : fx_val(Fx{at(sh.ph, (int)w1lo - 1), at(sh.po, (int)w1lo - 1)});
+    const double qd1 = all ? S : fx_val(Fx{at(sh.ph, (int)w1hi), at(sh.po, (int)w1hi)});
     const double tlo = u * (qd0 - delta) - delta, thi = u * (qd1 + delta) + delta;
     uint32_t b3 = DNB - 1, b4 = DNB - 1;
 #pragma unroll
@@ -335,7 +351,10 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
     w2hi = min(sh.q[PQ_B4], w1hi);
     w2lo = min(sh.q[PQ_B3], w2hi);
   }
-  if (w2hi + 1 >= w1lo) {  // touching or overlapping windows: one window
+  if (all) {  // the draw's window only
+    w1lo = w2lo;
+    w1hi = w2hi;
+  } else if (w2hi + 1 >= w1lo) {  // touching or overlapping windows: one window
     w2lo = min(w2lo, w1lo);
     w2hi = max(w2hi, w1hi);
     w1lo = w2lo;
@@ -354,7 +373,7 @@ __device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int
     const uint64_t x1o = sep ? at(sh.po, (int)w1lo - 1) - at(sh.po, (int)w2hi) : 0ull;
     const uint64_t xm[6] = {x0h, x0o, x1h, x1o, htot - x0h - x1h, otot - x0o - x1o};
     const uint32_t status =
-        (inw > 0 && inw <= (uint64_t)DCAP && S > 0.0 && fabsf(M) < INFINITY) ? DS_PLANNED : DS_FAIL;
+        (inw > 0 && inw <= (uint64_t)DCAP && S > 0.0 && fabsf(M) < INFINITY) ? (all ? DS_ALL : DS_PLANNED) : DS_FAIL;
     // the region counts and sums (read by the finish, which comes after this workgroup's pick ticket and so after
     // these stores), then the status and windows in one word, which the row's pick slices wait for
     st_ag(&ds->acc[DA_C0], n0);  // (the element counts of the regions the pick pass sums without listing)
@@ -480,6 +499,7 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
   const uint64_t pw = ld_ag(&ds->plan);
   const uint32_t w2hi = plan_win(pw, 1), w1lo = plan_win(pw, 2);
   const bool sep = w1lo > w2hi;  // an unlisted gap (region 1) between the draw window and the cut window
+  const bool all = plan_status(pw) == DS_ALL;
   const Fx X0{ld_ag(&ds->acc[DA_X0HI]), ld_ag(&ds->acc[DA_X0LO])}, X1{ld_ag(&ds->acc[DA_X1HI]), ld_ag(&ds->acc[DA_X1LO])};
   const Fx SF = fx_add(fx_add(X0, X1), Fx{ld_ag(&ds->acc[DA_RHI]), ld_ag(&ds->acc[DA_RLO])});
   const uint64_t c0 = ld_ag(&ds->acc[DA_C0]), c1 = ld_ag(&ds->acc[DA_C1]), tail = ld_ag(&ds->acc[DA_C2]);
@@ -700,12 +720,12 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
         good = r_s1 == rl + 1;
       } else {
         const uint64_t after = (!sep || g0) ? tail : c1 + tail;
-        good = after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp;
+        good = after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp || all;
       }
     }
     ok = good;
     if (ok) {
-      clast = fx_val(Al) / Sd;
+      clast = all && !inside ? 1.0 : fx_val(Al) / Sd;
       kkeep = sh.sub[last];
     }
     __syncthreads();  // (sh.pub, sh.sub before walk 1)
@@ -768,7 +788,7 @@ __device__ __forceinline__ double least_ge(double t, double S, bool &ok) {
 // acc: lane i holds the plan's acc[i].
 __device__ __forceinline__ void finish_wave(const FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab, int n,
                                          uint64_t e, uint64_t accv, int row, float Mf, double u, uint64_t K,
-                                         double topp, double minp, bool sep, uint32_t w1lo) {
+                                         double topp, double minp, bool sep, uint32_t w1lo, bool all) {
   const int l = lane_id();
   const bool val = l < n;
   const double M = (double)Mf;
@@ -817,9 +837,9 @@ __device__ __forceinline__ void finish_wave(const FinArgs a, DeepSlot *ds, FinSh
     Al = fx_add(fx_add(X0, Fx{rl64(ih, n - 1), rl64(il, n - 1)}), glast ? X1 : Fx{0, 0});
     const uint64_t rl = c0 + (uint64_t)last + (glast ? c1 : 0ull);
     const uint64_t after = (!sep || glast) ? tail : c1 + tail;  // unlisted elements ranked after the list
-    ok = after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp;
+    ok = after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp || all;
   }
-  const double clast = fx_val(Al) / Sd;
+  const double clast = all && fc < 0 ? 1.0 : fx_val(Al) / Sd;
   int32_t tok = -1;
   if (ok && a.mode == MODE_SAMPLE) {
     // the draw: the first kept entry whose inclusive prefix reaches u c_last; its exclusive prefix must lie below it
@@ -857,7 +877,7 @@ static_assert(FBN <= MT, "");
 // fixed-point masses gives every rank's exclusive prefix, and the cut and the draw are block minima. Five barriers.
 __device__ __forceinline__ void finish_block(const FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab, int n,
                                           uint64_t e, int row, float Mf, double u, uint64_t K, double topp,
-                                          double minp, bool sep, uint32_t w1lo) {
+                                          double minp, bool sep, uint32_t w1lo, bool all) {
   const int tid = threadIdx.x, l = lane_id(), w = tid >> 6;
   const bool val = tid < n;
   const double M = (double)Mf;
@@ -933,9 +953,9 @@ __device__ __forceinline__ void finish_block(const FinArgs a, DeepSlot *ds, FinS
     Al = fx_add(fx_add(X0, Fx{th, tl}), glast ? X1 : Fx{0, 0});
     const uint64_t rl = c0 + (uint64_t)last + (glast ? c1 : 0ull);
     const uint64_t after = (!sep || glast) ? tail : c1 + tail;  // unlisted elements ranked after the list
-    ok = ok && (after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp);
+    ok = ok && (after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp || all);
   }
-  const double clast = fx_val(Al) / Sd;
+  const double clast = all && fc == NONE ? 1.0 : fx_val(Al) / Sd;
   if (ok && a.mode == MODE_SAMPLE) {
     // the draw: the first kept entry whose inclusive prefix reaches u c_last; its exclusive prefix must lie below it.
     // Packed as rank << 1 | (not below).
@@ -983,14 +1003,14 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   if (spoil != 0u) return 0;  // (a slice gave up waiting for the plan: the exact path takes the row)
   if (nraw > (uint32_t)LC) return 1;
   const int n = (int)nraw;
-  const bool sep = w1lo > w2hi;
+  const bool sep = w1lo > w2hi, all = plan_status(pw) == DS_ALL;
   if (n <= WAVE) {  // one wave does it all, without a barrier
-    if (tid < WAVE) finish_wave(a, ds, sh, etab, n, v[0], accv, row, Mf, u, K, topp, minp, sep, w1lo);
+    if (tid < WAVE) finish_wave(a, ds, sh, etab, n, v[0], accv, row, Mf, u, K, topp, minp, sep, w1lo, all);
     return 0;
   }
   if (tid < DA_N) sh.acc[tid] = accv;  // (published by the first barrier of either path)
   if (n <= FBN) {
-    finish_block(a, ds, sh, etab, n, v[0], row, Mf, u, K, topp, minp, sep, w1lo);
+    finish_block(a, ds, sh, etab, n, v[0], row, Mf, u, K, topp, minp, sep, w1lo, all);
     return 0;
   }
   uint32_t *bcnt = reinterpret_cast<uint32_t *>(sh.sub), *bofs = bcnt + 2 * FB;
@@ -1173,9 +1193,9 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
     Al = fx_add(fx_add(X0, Fx{th, tl}), glast ? X1 : Fx{0, 0});
     const uint64_t rl = c0 + (uint64_t)last + (glast ? c1 : 0ull);
     const uint64_t after = (!sep || glast) ? tail : c1 + tail;  // unlisted elements ranked after the list
-    ok = ok && (after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp);
+    ok = ok && (after == 0 || rl + 1 >= K || fx_val(Al) / Sd >= topp || all);
   }
-  const double clast = fx_val(Al) / Sd;
+  const double clast = all && fc == NONE ? 1.0 : fx_val(Al) / Sd;
   if (ok && a.mode == MODE_SAMPLE) {
     // the draw: the first kept entry whose inclusive prefix reaches u c_last; its exclusive prefix must lie below it
     // (else the draw falls in an unlisted region: before the list, or in the gap). Packed as rank << 1 | (not below).
@@ -1398,7 +1418,7 @@ __device__ __forceinline__ int pick_item(const ScanArgs &a, int slot, int slice,
     }
     __syncthreads();
     const uint64_t pw = sh.pplan;
-    planned = plan_status(pw) == DS_PLANNED;
+    planned = plan_status(pw) == DS_PLANNED || plan_status(pw) == DS_ALL;
     if (planned) {
       w2lo = plan_win(pw, 0);
       w2hi = plan_win(pw, 1);

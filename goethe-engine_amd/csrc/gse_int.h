@@ -76,10 +76,12 @@ static_assert(sizeof(SliceRec) == 64, "");
 constexpr int DEEP_MAX = 1024;  // split-row slots at most (a handle has min(max_rows, DEEP_MAX); more deep rows: the
                                 // exact path takes them)
 constexpr int DSMAX = 64;      // slices per deep row, at most
-constexpr int DNB = 512;       // histogram bins of d = z_max - z, 1/32 wide (the last one open-ended)
+constexpr int DNB = 512;       // histogram bins of d = z_max - z: 1/32 wide to d = 12, then wider (gse_deep.hip)
 constexpr int DCAP = 8192;     // window elements listed per deep row
 
-enum : uint32_t { DS_PENDING = 0u, DS_PLANNED = 1u, DS_FAIL = 2u };
+// DS_ALL: planned, and every element is kept (a sampled row with no top-p, top-k or min-p cut): the list holds the draw's
+// window only.
+enum : uint32_t { DS_PENDING = 0u, DS_PLANNED = 1u, DS_FAIL = 2u, DS_ALL = 3u };
 
 // DeepSlot::plan: the status in bits 0-7, then the windows w2lo, w2hi, w1lo, w1hi (inclusive bins, 12 bits each).
 __host__ __device__ constexpr uint64_t plan_word(uint32_t st, uint32_t w2lo, uint32_t w2hi, uint32_t w1lo,
