@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <new>
 #include <string>
@@ -197,6 +198,10 @@ gse::ScanArgs make_args(gse_handle *h, const gse_batch &b, int mode) {
   parts(h, b.rows, b.vocab, plain ? (uint32_t)gse::PTOK_PLAIN : (uint32_t)gse::PTOK, &a.nparts, &a.plen);
   a.kt = a.plen > gse::PTOK ? (int)(((int64_t)gse::KT * a.plen + gse::PTOK - 1) / gse::PTOK)
                             : plain ? gse::KT : gse::KT_HM;
+  const bool many = a.nparts > gse::KT_PARTS;  // (rows of many parts share out the listing targets)
+  if (many) a.kt = std::max(gse::KT_MIN, a.kt * gse::KT_SHARE / a.nparts);
+  a.kshare = 256 * std::min((many ? gse::KT_SHARE : gse::KT_TOPK), a.nparts) / a.nparts;
+  a.kmin = many ? gse::KT_MIN : gse::KT_MINK;
   a.vfirst = (int)((int64_t)gse::CAPW / 4 * a.kt / gse::KT_VALVE) + 1;
   a.mode = mode;
   a.xcd_map = 1;

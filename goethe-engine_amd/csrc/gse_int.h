@@ -52,6 +52,19 @@ constexpr int PTOK_PLAIN = 131072;  // tokens per part, at most, in a call with 
 constexpr int KT = 200;       // tokens of a part of at most PTOK tokens its listing threshold aims to leave above it
 constexpr int KT_HM = 150;    // the same in a call with histories or masks: its rows' heads certify with shorter lists,
                               // which the resolve gathers and sorts faster (much lower and some rows need the exact path)
+constexpr int KT_PARTS = 4;   // a row of more parts shares out the targets of KT_SHARE of them: each part lists its own
+constexpr int KT_SHARE = 3;   // candidates, and 16 to 32 parts at the full target listed 3200 to 6400 entries, which the
+constexpr int KT_MIN = 24;    // resolve gathers and which overflow its head (2048); not below KT_MIN a part. One bf16 row
+                              // of 128256 (16 parts) 43.9 -> 25.6 us, 64 rows of 151936 (16 parts) 88 -> 33.6 us; shares of
+                              // 4, 3, 2 parts: 27.0, 25.6, 24.3 us and 35.8, 33.6, 31.9 us, but 32 rows with every cut
+                              // 57.3, 56.8, 61.0 us (more rows past their heads); at 4 parts a row (256 rows of 151936) the
+                              // full target stays: 99.7 us, 101.9 with 3/4 of it
+// Rows with top-k keep at most top_k elements, whichever parts hold them: from KT_TOPK parts on, the parts share KT_TOPK
+// times 2 top_k + 32 (rows of more than KT_PARTS parts KT_SHARE times it), each at least KT_MINK (KT_MIN). 8 rows of 32000
+// (3 parts, top-k 40) 28.6 -> 27.5 us, 256 rows of 151936 with every cut 98.5 -> 97.5 us; least targets of 32, 48, 64 with
+// 4 parts: 98.3, 97.5, 97.5 us; the same share with 16 parts and 48 cost 4 rows 28.1 -> 32.8 us.
+constexpr int KT_TOPK = 2;
+constexpr int KT_MINK = 48;
 constexpr int KT_VALVE = 222; // the listing target at which a part's first-chunk valve is CAPW / 4 (scaled with kt)
 constexpr int PCHUNK = 1024;  // part lengths are multiples of this (one wave chunk)
 constexpr int PMIN = 8192;    // tokens per part, at least, when a small batch is split to fill the device: every part
@@ -136,6 +149,7 @@ struct ScanArgs {
   int64_t ld;
   int dtype, V, rows, nch, mode, force_exact, xcd_map;
   int nparts, plen;  // the main pass: parts per row, tokens per part (a multiple of 1024; the last part may be shorter)
+  int kshare, kmin;  // rows with top-k: a part's share of 2 top_k + 32 in 1/256, and its least target
   int kt, vfirst;    // tokens of a part its listing threshold aims to leave above it; list length that first opens the valve
   int pmajor;        // workgroup L streams part L / rows8 of row L % rows8 (else the parts of a row are consecutive)
   const gse_row *params;

@@ -116,7 +116,12 @@ __device__ __forceinline__ void set_hard(const ScanArgs &a, RowInfo *ri, uint64_
 // ---------------------------------------------------------------------------------------------------------------------
 // Row resolve, run by the last workgroup of the row.
 
-enum { EV_DONE = 0, EV_MORE = 1, EV_HARD = 2 };
+enum { EV_DONE = 0, EV_HARD = 1 };
+// The least share of the mass that top-p keeps that the head must hold for the row's draw to be looked for in it. In a
+// flatter row few draws fall there, and a batch of such rows needs the split-row pass for the others anyway: skipping
+// their sort and evaluation keeps the main pass's tail short.
+constexpr double HEAD_DRAW = 0.25;
+constexpr uint32_t NONE = 0xFFFFFFFFu;
 
 struct RowEval {
   const ScanArgs *a;
@@ -141,8 +146,8 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
   const int n = ev.n;
   if (ev.nlp > n) return EV_HARD;  // logprobs past the finite elements: -inf ranks in id order
   if (tid == 0) {
-    sh.mfail_sure = 0xFFFFFFFFu;
-    sh.mfail_maybe = 0xFFFFFFFFu;
+    sh.mfail_sure = NONE;
+    sh.mfail_maybe = NONE;
     sh.jcount = 0;
   }
   // Exact masses e_r of the sorted ranks, then their inclusive prefixes I_r in place (in LDS). Wave w takes ranks
@@ -210,7 +215,7 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
   const double topp = P.top_p, minp = P.min_p;
   const double B = ev.B + 2e-15 * Sm;
   const double q0 = 1.0 / Sm, tlo = topp * (Sm - B), thi = topp * (Sm + B);
-  uint32_t fsure = 0xFFFFFFFFu, fmaybe = 0xFFFFFFFFu;
+  uint32_t fsure = NONE, fmaybe = NONE;
 #pragma unroll 1
   for (int s = 0; s < RPW / WAVE; ++s) {
     const int r = w * RPW + s * WAVE + lane;
@@ -223,8 +228,8 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
         km = e >= minp;
         if (fabs(e - minp) <= 1e-12 * minp) km = e / Sm >= minp * q0;
       }
-      if ((!kk || !km || A >= thi) && fsure == 0xFFFFFFFFu) fsure = (uint32_t)r;
-      if ((!kk || !km || !(A < tlo)) && fmaybe == 0xFFFFFFFFu) fmaybe = (uint32_t)r;
+      if ((!kk || !km || A >= thi) && fsure == NONE) fsure = (uint32_t)r;
+      if ((!kk || !km || !(A < tlo)) && fmaybe == NONE) fmaybe = (uint32_t)r;
     }
   }
   fsure = wave_min_u32(fsure);
@@ -234,12 +239,37 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
     atomicMin(&sh.mfail_maybe, fmaybe);
   }
   __syncthreads();
-  uint32_t m = sh.mfail_sure;
-  if (m != sh.mfail_maybe) return EV_HARD;
-  if (m == 0xFFFFFFFFu) {  // every rank of the head is kept
-    if (!ev.complete) return EV_HARD;  // the keep prefix runs past the certified head
-    m = (uint32_t)n;
+  // m1 <= m2, NONE past the head. Settled: the cut is one rank of the head, or the head is the whole row and all of it is
+  // kept.
+  const uint32_t m1 = sh.mfail_maybe, m2 = sh.mfail_sure;
+  if (__builtin_expect(m1 != m2 || (m1 == NONE && !ev.complete), 0)) {
+    // An unsettled cut still leaves the draw to the head when every c_last it allows puts u c_last between the same two
+    // prefixes. c_last is at least the prefix of the first rank that may fail, or, past the head, the head's mass and
+    // (top-p the only cut) top_p S; at most the prefix of the first that surely fails, or top_p S and one element more
+    // (the last kept one, at most the head's last), or S. Only a token is wanted: dist and verify nodes that take
+    // dist + mss need the boundary itself.
+    if (n == 0 || a.mode != MODE_SAMPLE || (a.tree && (P.flags & GSE_ROW_MSS)) || htot < HEAD_DRAW * topp * Sm)
+      return EV_HARD;
+    const double clo = m1 != NONE ? ee[m1 - 1] : P.top_k > 0 || minp > 0.0 ? htot : fmax(htot, tlo);
+    const double chi = m2 != NONE ? ee[m2 - 1] : fmin(Sm + B, thi + (n > 1 ? ee[n - 1] - ee[n - 2] : htot));
+    const double u = a.uni ? a.uni[ev.row] : uniform64(P.seed, P.idx), mar = 1e-13 * Sm;  // (far above the prefixes' roundings)
+    const double tl = u * clo - mar, th = u * chi + mar;
+    uint32_t cnt = 0;  // (the counts below either threshold, 16 bits each: n <= 2048)
+#pragma unroll 1
+    for (int r = tid; r < n; r += MT) cnt += (ee[r] < tl ? 1u : 0u) + (ee[r] < th ? 0x10000u : 0u);
+    cnt = wave_sum_u32(cnt);
+    if (lane == 0 && cnt) atomicAdd(&sh.jcount, cnt);
+    __syncthreads();
+    const uint32_t jl = sh.jcount & 0xFFFFu, jh = sh.jcount >> 16;
+    if (jl != jh || jl >= (m1 != NONE ? m1 : (uint32_t)n)) return EV_HARD;
+    if (tid == 0) {
+      const int32_t tok = (int32_t)pk_id(arr[jl]);
+      set_info(ri, arr[0], 0ull, Sm, 0.0, R_DONE, tok);
+      a.tokens[ev.row] = tok;
+    }
+    return EV_DONE;
   }
+  const uint32_t m = m1 != NONE ? m1 : (uint32_t)n;
   // c_last = I_{m-1}; j = #{r < m : I_r < u c_last}, clamped to [0, m - 1] (sampling.py:81-83)
   const double clast = ee[m - 1];
   int32_t tok = -1;
@@ -552,6 +582,12 @@ __device__ __forceinline__ void resolve_row(const ScanArgs &a, int row, const gs
       const double hhi = h * (1.0 + 1e-11), hlo = h * (1.0 - 1e-11);
       const double B = ev.B + 2e-15 * (ev.S + hhi);
       past = hhi < P.top_p * (ev.S + hlo - B);
+      // (unless the draw surely falls inside the head: c_last is at most S, and top_p S and one unlisted element)
+      if (past && a.mode == MODE_SAMPLE && !(a.tree && (P.flags & GSE_ROW_MSS)) && h >= HEAD_DRAW * P.top_p * (ev.S + h)) {
+        const double u = a.uni ? a.uni[row] : uniform64(P.seed, P.idx);
+        const double ek = exp_nonpos((double)fkey_inv(kappa) - M, sh.etab), Sh = ev.S + hhi + B;
+        past = !(u * fmin(Sh, P.top_p * Sh + ek) < hlo);
+      }
     }
     if (!past) {
       sort_head(sh, n, mk, kappa);
@@ -923,11 +959,13 @@ __device__ __forceinline__ float fmax_q(float a, float b) {
 
 // Raises the wave's listing threshold to the x key k (uniform): xt = the value of k, R = z(xt), and the lanes' sums
 // rescaled to the new reference (fp64). c0 = RN(-R log2(e)); an R whose c0 leaves the fp32 range (|R| > 2.3e38) marks
-// the part (its row takes the split-row finish or the exact path). An R of -inf leaves only -inf elements unlisted, of
-// mass 0: c0 = -inf gives them exp2(-256) = 0.
+// the part (its row takes the split-row finish or the exact path). The lowest threshold, which leaves only -inf elements
+// unlisted (a part whose sample has no allowed token), has R = -inf, not its own value -FLT_MAX (whose c0 would mark the
+// part: every masked row of such a part with T = 1, or greedy with logprobs, then went on, the latter to the exact path,
+// 390 us for 16 rows of 151936): their mass is 0, c0 = -inf gives them exp2(-256) = 0.
 __device__ __forceinline__ void set_threshold(Run &rn, uint32_t k, bool divide, double Rd) {
   const float xt = fkey_inv(k);
-  const float R = divide ? div_exact(xt, Rd) : xt;
+  const float R = k <= KEY_NEGINF + 1u ? -INFINITY : divide ? div_exact(xt, Rd) : xt;
   if (rn.R > -INFINITY && R > rn.R) {
     const double f = exp((double)rn.R - (double)R);
     rn.s *= f;
@@ -1172,8 +1210,8 @@ __device__ __forceinline__ bool part_body(const ScanArgs &a, const gse_row &P, c
     // The listing threshold: the rank-kp largest of the 256 lane maxima of the waves' first chunks (a 2048-token
     // sample). kp is scaled so that about T tokens of the part lie above it: kp = T * (allowed tokens in the sample) /
     // (allowed tokens in the part), counted exactly, so that a mask whose allowed tokens cluster in runs does not skew
-    // it. T = a.kt (200 for a part of at most PTOK tokens, 150 in a call with histories or masks), or 2 top_k + 32 (at
-    // most 2 a.kt) for rows that keep at most top_k elements.
+    // it. T = a.kt (200 for a part of at most PTOK tokens, 150 in a call with histories or masks, less for rows of many
+    // parts), or a share of 2 top_k + 32 (at most 2 a.kt) for rows that keep at most top_k elements.
     uint32_t as = 0;
 #pragma unroll
     for (int i = 0; i < EPL; ++i) as += x0[i] > -INFINITY ? 1u : 0u;
@@ -1194,7 +1232,8 @@ __device__ __forceinline__ bool part_body(const ScanArgs &a, const gse_row &P, c
       Ap += sh.wflags[q];
     }
     const uint32_t kt = (uint32_t)a.kt;
-    const uint32_t T = P.top_k > 0 ? min(2u * kt, (uint32_t)(2 * max(P.top_k, nlp_of(a, P)) + 32)) : kt;
+    const uint32_t tk = (uint32_t)(2 * max(min(P.top_k, 4096), nlp_of(a, P)) + 32) * (uint32_t)a.kshare >> 8;
+    const uint32_t T = P.top_k > 0 ? min(2u * kt, max(tk, (uint32_t)a.kmin)) : kt;
     // (a sample with few allowed tokens estimates nothing: then the lowest lane maximum, and the valve bounds the lists)
     const uint32_t kp = As < 16u ? max(act, 1u) : max(1u, min(act, (T * As + Ap - 1) / max(Ap, 1u)));  // (T As < 2^22)
     uint32_t r = 0;

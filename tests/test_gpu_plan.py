@@ -66,3 +66,57 @@ def test_dist_of_long_tails(ge, gpu):
     assert (paths == ge._lib.PATH_EXACT).sum() == 0, paths
     for r in range(n):
         np.testing.assert_allclose(d[r], ora.dist(x[r], params[r]), rtol=1e-12, atol=1e-300)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_draws_settled_in_the_head(ge, gpu, dtype):
+    """Rows whose keep set runs past the certified head but whose draw mostly falls inside it: small batches over one
+    long vocabulary (many parts a row) and larger ones, every cut alone and together, uniforms from 0 to just below 1.
+    Tokens against the oracle on both paths; most rows end in the main pass."""
+    v = 100003
+    rng = np.random.default_rng(31)
+    P = ge.sampling.SamplingParams
+    cuts = [dict(top_p=0.9), dict(top_p=0.97), dict(), dict(top_k=3000, top_p=0.999), dict(min_p=1e-4),
+            dict(top_k=400, top_p=0.95, min_p=1e-3)]
+    us = [0.0, 2.0 ** -53, 0.1, 0.5, 0.75, 0.9, 0.97, 1.0 - 2.0 ** -53]
+    for n in (1, 6, 48):
+        main = 0
+        for rep in range(8 if n == 1 else 1):
+            x = torch.from_numpy(_zipf(rng, n, v))
+            x = x.bfloat16() if dtype == "bf16" else x
+            params = [P(temperature=[0.7, 1.0, 1.3][(r + rep) % 3], **cuts[(r + rep) % 6]) for r in range(n)]
+            u = np.array([us[(r // 2 + rep) % 8] for r in range(n)])
+            sel = ge.sampling.sample_ex(x.to(gpu), params, None, None, None, uniforms=u)
+            paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
+            assert sel.tolist() == ora.sample(x.float().numpy(), params, None, None, None, uniforms=u), (n, rep)
+            main += int((paths == ge._lib.PATH_MAIN).sum())
+        assert main >= (4 if n == 1 else n // 2), (n, main)
+
+
+def test_masked_rows_whose_samples_are_empty(ge, gpu):
+    """Masked rows whose allowed runs lie outside most parts' samples (those parts start listing everything). Greedy rows
+    with logprobs, sampled rows with and without, T = 1 and not: tokens, ids and logprobs against the oracle, none on the
+    exact path."""
+    v, n = 151936, 12
+    rng = np.random.default_rng(8)
+    x = rng.normal(0.0, 2.0, size=(n, v)).astype(np.float32)
+    masks = np.zeros((n, v), bool)
+    for r in range(n):
+        for s in range(18):  # (runs of 400 tokens past the first 2048 of every 8192)
+            masks[r, s * 8192 + 4000 + 7 * r:s * 8192 + 4400 + 7 * r] = True
+    P = ge.sampling.SamplingParams
+    params = [[P(logprobs=7), P(temperature=1.0, top_p=0.9, logprobs=20), P(temperature=0.8, top_k=50)][r % 3]
+              for r in range(n)]
+    u = rng.random(n)
+    sel = ge.sampling.sample_ex(torch.from_numpy(x).to(gpu), params, None, None, [torch.from_numpy(m) for m in masks],
+                                uniforms=u)
+    paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
+    want = ora.sample_full(x, params, None, None, list(masks), None, u)
+    assert sel.tolist() == [w["token"] for w in want]
+    ids, lps = sel.logprob_ids.cpu().numpy(), sel.logprobs.cpu().numpy()
+    for r in range(n):
+        if params[r].logprobs:
+            k = params[r].logprobs
+            assert list(ids[r, :k]) == list(want[r]["logprob_ids"])
+            np.testing.assert_allclose(lps[r, :k], want[r]["logprobs"], rtol=2e-7)
+    assert (paths == ge._lib.PATH_EXACT).sum() == 0, paths
