@@ -444,30 +444,17 @@ __device__ __forceinline__ void excl_scan2(uint64_t &a, uint64_t &b, uint64_t &t
   __syncthreads();
 }
 
-// Sorts sh.sub[0, n) descending (bitonic over the next power of two, zero padded). Rolled loops: it runs once per
-// row, cold, so its code is kept small.
+// Sorts sh.sub[0, n), n <= MT, descending: thread t ranks entry t by the count of greater ones (two barriers, where a
+// bitonic network of 64 entries has 21).
 __device__ __forceinline__ void sort_sub(int n, FinShared &sh) {
   const int tid = threadIdx.x;
-  int N = 2;
-  while (N < n) N <<= 1;
-  for (int i = n + tid; i < N; i += MT) sh.sub[i] = 0ull;
+  const uint64_t e = tid < n ? sh.sub[tid] : 0ull;
+  int r = 0;
+#pragma unroll 4
+  for (int q = 0; q < n; ++q) r += sh.sub[q] > e ? 1 : 0;
   __syncthreads();
-#pragma unroll 1
-  for (int k = 2; k <= N; k <<= 1) {
-#pragma unroll 1
-    for (int j = k >> 1; j > 0; j >>= 1) {
-#pragma unroll 1
-      for (int i = tid; i < N / 2; i += MT) {
-        const int lo = ((i & ~(j - 1)) << 1) | (i & (j - 1)), hi = lo + j;
-        const uint64_t x = sh.sub[lo], y = sh.sub[hi];
-        if ((lo & k) == 0 ? x < y : x > y) {
-          sh.sub[lo] = y;
-          sh.sub[hi] = x;
-        }
-      }
-      __syncthreads();
-    }
-  }
+  if (tid < n) sh.sub[r] = e;
+  __syncthreads();
 }
 
 // Sub-bin of a window entry.
@@ -520,7 +507,23 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
 #pragma unroll
     for (int j = 0; j < LC / MT; ++j) sh.lc[j * MT + tid] = v[j];
   }
-  auto entry = [&](int i) -> uint64_t { return i < LC ? sh.lc[i] : ld_ag(&lst[i]); };
+  // f of every entry, LC at a time: the first LC from LDS, then rounds of loads issued together (a load at a time, each
+  // waited for, four passes over a list of 4000 entries took 60 us)
+  auto each_entry = [&](auto f) __attribute__((always_inline)) {
+    constexpr int EB = LC / MT;
+#pragma unroll 1
+    for (int b = 0; b < n; b += LC) {
+      uint64_t v[EB];
+#pragma unroll
+      for (int j = 0; j < EB; ++j) {
+        const int i = b + j * MT + tid;
+        v[j] = b == 0 ? sh.lc[i] : ld_ag(&lst[min(i, DCAP - 1)]);
+      }
+#pragma unroll
+      for (int j = 0; j < EB; ++j)
+        if (b + j * MT + tid < n) f(v[j]);
+    }
+  };
   // key ranges of the two windows
   if (tid < 2) {
     sh.kmax[tid] = 0;
@@ -533,12 +536,14 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
   __syncthreads();
   {
     uint32_t kx[2] = {0u, 0u}, kn[2] = {NONE, NONE};
-    for (int i = tid; i < n; i += MT) {
-      const uint32_t k = pk_key(entry(i));
-      const int g = (sep && dbin(fkey_inv(k), Mf) >= w1lo) ? 1 : 0;
-      kx[g] = max(kx[g], k);
-      kn[g] = min(kn[g], k);
-    }
+    each_entry([&](uint64_t e) __attribute__((always_inline)) {
+      const uint32_t k = pk_key(e);
+      const bool g = sep && dbin(fkey_inv(k), Mf) >= w1lo;
+      kx[0] = max(kx[0], g ? 0u : k);
+      kn[0] = min(kn[0], g ? NONE : k);
+      kx[1] = max(kx[1], g ? k : 0u);
+      kn[1] = min(kn[1], g ? k : NONE);
+    });
     for (int g = 0; g < 2; ++g) {  // (one LDS atomic per wave)
       kx[g] = wave_max_u32(kx[g]);
       kn[g] = wave_min_u32(kn[g]);
@@ -557,15 +562,15 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
     shift[g] = sft;
   }
   // exact sub-bin counts, masses and head keys
-  for (int i = tid; i < n; i += MT) {
-    const uint32_t k = pk_key(entry(i));
+  each_entry([&](uint64_t e) __attribute__((always_inline)) {
+    const uint32_t k = pk_key(e);
     const int b = sub_of(k, shift, sep, w1lo, Mf, sh);
     const Fx f = mass_of(k, M, etab);
     atomicAdd(&sh.scnt[b], 1u);
     atomicMax(&sh.stop[b], k);
     atomicAdd((unsigned long long *)&sh.shi[b], (unsigned long long)f.hi);
     atomicAdd((unsigned long long *)&sh.slo[b], (unsigned long long)f.lo);
-  }
+  });
   __syncthreads();
   // exclusive prefix over sub-bins (thread t = sub-bin t, in key order): rank and mass at each sub-bin head
   const uint32_t mycnt = sh.scnt[tid], mytop = sh.stop[tid];
@@ -648,20 +653,29 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
     }
     if (tid == 0) sh.ns = 0;
     __syncthreads();
-    for (int i = tid; i < n; i += MT) {
-      const uint64_t pk = entry(i);
+    each_entry([&](uint64_t pk) __attribute__((always_inline)) {
       if (sub_of(pk_key(pk), shift, sep, w1lo, Mf, sh) == sb) {
         const uint32_t pos = atomicAdd(&sh.ns, 1u);
         if (pos < (uint32_t)SUBC) sh.sub[pos] = pk;
       }
-    }
+    });
     __syncthreads();
     if (sh.ns != cnt) {
       ok = false;
       break;
     }
     const int m = (int)cnt;
-    sort_sub(m, sh);
+    if (m <= MT) {
+      sort_sub(m, sh);
+    } else {  // (a tie group, mostly: in registers, then the first LC entries, whose LDS it used, again)
+      sort_lds_regs<SW>(sh.sub, sh.lc, m);
+      uint64_t v[LC / MT];
+#pragma unroll
+      for (int j = 0; j < LC / MT; ++j) v[j] = ld_ag(&lst[j * MT + tid]);
+#pragma unroll
+      for (int j = 0; j < LC / MT; ++j) sh.lc[j * MT + tid] = v[j];
+      __syncthreads();
+    }
     // exclusive prefix at entry tid * SW, then the first entry that meets the walk's test
     uint64_t hi = 0, lo = 0, thi, tlo;
 #pragma unroll 1
@@ -754,6 +768,7 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
 // and one block minimum each. The unlisted region between the windows (X1, c1 elements) counts before the cut
 // window's entries. The tests and fixed-point sums are finish_row's; a failed check leaves the row to the exact path.
 constexpr int FB = 1024;  // key buckets per window
+constexpr int FBK = 64;   // the largest bucket whose members are ranked by counting
 static_assert(2 * 2 * FB * sizeof(uint32_t) <= SUBC * sizeof(uint64_t), "bucket counts and starts live in sub");
 static_assert(SUBC >= LC, "masses by rank live in sub");
 
@@ -1016,7 +1031,7 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   uint32_t *bcnt = reinterpret_cast<uint32_t *>(sh.sub), *bofs = bcnt + 2 * FB;
   double *msr = reinterpret_cast<double *>(sh.sub);  // (after the ranks: the masses by rank)
   for (int b = tid; b < 2 * FB; b += MT) bcnt[b] = 0;
-  if (tid < 2) sh.q[tid] = NONE;
+  if (tid < 3) sh.q[tid] = tid < 2 ? NONE : 0u;
   // each entry's window and the key range of each window (per-wave ranges in wred / wred2, no atomics)
   uint32_t gm = 0, kx0 = 0, kx1 = 0, kn0 = NONE, kn1 = NONE;
 #pragma unroll
@@ -1071,12 +1086,15 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   // bucket starts: thread t owns buckets [8 t, 8 t + 8)
   {
     constexpr int BT = 2 * FB / MT;
-    uint32_t c[BT], loc = 0;
+    uint32_t c[BT], loc = 0, mx = 0;
 #pragma unroll
     for (int j = 0; j < BT; ++j) {
       c[j] = bcnt[tid * BT + j];
       loc += c[j];
+      mx = max(mx, c[j]);
     }
+    mx = wave_max_u32(mx);
+    if (lane_id() == 0) atomicMax(&sh.q[2], mx);
     const uint32_t inc = wave_incl_scan_u32(loc);
     if (lane_id() == WAVE - 1) sh.wsum[w] = inc;
     __syncthreads();
@@ -1090,6 +1108,10 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   }
   __syncthreads();
   const uint32_t n0 = sep ? bofs[FB] : (uint32_t)n;  // entries of the draw window (they rank first)
+  // A crowded bucket (a tie group: bf16 logits) goes to the sub-bin walk, which sorts only the groups that hold the cut and
+  // the draw: ranking its members against each other reads them all once per member (one bf16 row of 151936 tokens: 67
+  // us; sorting the whole list in registers 66; the walk 61).
+  if (sh.q[2] > (uint32_t)FBK) return 1;
 #pragma unroll
   for (int j = 0; j < SP; ++j)
     if (j * MT + tid < n) sh.lc[bofs[bucket(j)] + sl[j]] = v[j];
@@ -1327,6 +1349,11 @@ __device__ __noinline__ void exact_rows(bool scan) {
   }
 }
 
+// A verify node that takes dist + mss wants dist's keep boundary, not a draw.
+__device__ __forceinline__ int row_mode(const ScanArgs &a, const gse_row &P) {
+  return a.tree && (P.flags & GSE_ROW_MSS) ? (int)MODE_DIST : a.mode;
+}
+
 template <int DT, bool AL>
 __device__ __forceinline__ void count_item(const ScanArgs &a, int slot, int slice, const DGeom &g, PickShared &ps,
                                            const double *etab) {
@@ -1371,7 +1398,7 @@ __device__ __forceinline__ void count_item(const ScanArgs &a, int slot, int slic
   __syncthreads();  // (every thread has read the ticket: the plan's tables reuse the slice's LDS)
   if (!lastc) return;
   __builtin_amdgcn_s_setprio(3);  // (the row's other slices wait for the plan)
-  plan_block(gh, ds, a.mode, ps.p.pl);
+  plan_block(gh, ds, row_mode(a, P), ps.p.pl);
   if (tid == 0) {
     ds->cdone = 0u;
     g_pl[slot >> 6] |= 1ull << (slot & 63);  // (its pick item takes the rows-planned ticket)
@@ -1481,7 +1508,7 @@ __device__ __forceinline__ void finish_item(const ScanArgs &a, int fs, PickShare
   __builtin_amdgcn_s_setprio(3);  // (the finish is the row's critical path)
   if (tid == 0) g_fin = 0u;
   if (planned) {
-    const FinArgs fa{a.dlist + (size_t)slot * DCAP, a.info, a.tokens, a.mode};
+    const FinArgs fa{a.dlist + (size_t)slot * DCAP, a.info, a.tokens, row_mode(a, ds->P)};
     if (a.fin_sorted ? finish_sorted(fa, ds, ps.f, etab) != 0 : ld_ag(&ds->spoil) == 0u) {
       finish_row(fa, ds, ps.f, etab);
     }

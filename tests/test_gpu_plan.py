@@ -120,3 +120,23 @@ def test_masked_rows_whose_samples_are_empty(ge, gpu):
             assert list(ids[r, :k]) == list(want[r]["logprob_ids"])
             np.testing.assert_allclose(lps[r, :k], want[r]["logprobs"], rtol=2e-7)
     assert (paths == ge._lib.PATH_EXACT).sum() == 0, paths
+
+
+@pytest.mark.parametrize("flags", [0, 16])
+@pytest.mark.parametrize("v", [9001, 50257, 151936])
+def test_window_lists_of_ties(ge, gpu, v, flags):
+    """Flat rows with tie groups of tens to thousands of elements at the cut and at the draw (bf16 logits; fp32 logits on
+    a grid), so that the window lists are long and their key buckets crowded: tokens against the oracle, by the sorted
+    finish and by the sub-bin walk (GSE_BATCH_SUBBIN_FINISH)."""
+    assert ge._lib.BATCH_SUBBIN_FINISH == 16
+    n = 16
+    rng = np.random.default_rng(v)
+    P = ge.sampling.SamplingParams
+    params = [P(temperature=[1.0, 0.7, 1.6, 1.0][r % 4], top_p=[0.95, 0.8, 1.0, 0.999][r // 4], min_p=[0.0, 0.03][r % 2])
+              for r in range(n)]
+    base = rng.normal(0.0, 2.0, size=(n, v)).astype(np.float32)
+    u = np.array([ora.uniform(r, 11) for r in range(n)], np.float64)
+    for x in (torch.from_numpy(base).bfloat16(), torch.from_numpy(np.round(base * 16) / 16),
+              torch.from_numpy(np.round(base * 64) / 64)):
+        sel = ge.sampling.sample_ex(x.to(gpu), params, None, None, None, uniforms=u, flags=flags)
+        assert sel.tolist() == ora.sample(x.float().numpy(), params, None, None, None, uniforms=u)
