@@ -49,8 +49,14 @@ def mss_batch(p, kids, seeds, idxs):
     pt = pt.to(dev, torch.float64).reshape(len(kids), -1).clone()
     n, v = pt.shape
     kmax = max([len(k) for k in kids] + [1])
-    ktok = np.full((n, kmax), -1, np.int32)
-    kq = np.full((n, kmax), -1, np.int32)
+    # one host buffer and one copy for the kids, seeds and indexes, and one copy back for the answers: each small
+    # synchronous copy is 8 to 13 us of host time (one node, dist + mss through Python: 175 -> 111 us)
+    host = np.empty(4 * n + 2 * n * kmax, np.int32)
+    host[:2 * n].view(np.uint64)[:] = [int(s) & M64 for s in seeds][:n]
+    host[2 * n:4 * n].view(np.uint64)[:] = [int(i) & M64 for i in idxs][:n]
+    ktok, kq = host[4 * n:4 * n + n * kmax].reshape(n, kmax), host[4 * n + n * kmax:].reshape(n, kmax)
+    ktok[:] = -1
+    kq[:] = -1
     qs = []
     for a, ks in enumerate(kids):
         for r, (x, q) in enumerate(ks):
@@ -62,24 +68,21 @@ def mss_batch(p, kids, seeds, idxs):
                 qs.append(q)
     qt = _f64_rows(qs, dev)
     h = _lib.handle(dev.index, 1, v)
-    ktok_d = torch.from_numpy(ktok).to(dev)
-    kq_d = torch.from_numpy(kq).to(dev)
-    seed_d, idx_d = _u64(seeds, dev), _u64(idxs, dev)
-    otok = torch.empty(n, dtype=torch.int32, device=dev)
-    okid = torch.empty(n, dtype=torch.int32, device=dev)
+    arg = torch.from_numpy(host).to(dev)
+    at = arg.data_ptr()
+    out = torch.empty((2, n), dtype=torch.int32, device=dev)
     b = _lib.MssBatch()
     b.size = C.sizeof(_lib.MssBatch)
     b.nodes, b.vocab, b.max_kids = n, v, kmax
     b.p, b.p_ld = pt.data_ptr(), pt.stride(0)
     b.q, b.q_ld = (qt.data_ptr(), qt.stride(0)) if qt is not None else (None, v)
-    b.kid_tok, b.kid_q = ktok_d.data_ptr(), kq_d.data_ptr()
-    b.seed, b.idx = seed_d.data_ptr(), idx_d.data_ptr()
-    b.out_token, b.out_kid = otok.data_ptr(), okid.data_ptr()
+    b.seed, b.idx = at, at + 8 * n
+    b.kid_tok, b.kid_q = at + 16 * n, at + 16 * n + 4 * n * kmax
+    b.out_token, b.out_kid = out.data_ptr(), out.data_ptr() + 4 * n
     b.stream = torch.cuda.current_stream(dev).cuda_stream
     h.call("gse_mss", C.byref(b))
-    toks = otok.cpu().tolist()
-    kid = [None if k < 0 else int(k) for k in okid.cpu().tolist()]
-    return [int(t) for t in toks], kid
+    toks, kid = out.cpu().tolist()
+    return toks, [None if k < 0 else k for k in kid]
 
 
 def mss(p, kids, seed, i):
