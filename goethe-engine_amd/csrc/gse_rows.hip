@@ -371,6 +371,7 @@ __global__ __launch_bounds__(RT) void mss_kernel(MssArgs a) {
         nd.next = (uint32_t)(D + 1);
       }
     } else {
+      __syncthreads();  // (every wave has read p[kn.x], which the loop writes)
       for (int t = tid; t < V; t += RT) {
         const double v = at(t);
         p[t] = total > 0.0 ? v / total : v;

@@ -70,6 +70,35 @@ def test_mss_sizes(ge, gpu, v):
         assert max(levels) == 5, levels  # a node whose five kids were all rejected
 
 
+@pytest.mark.parametrize("v", [200, 5000, 50257])
+def test_mss_kids_past_the_sliced_levels(ge, gpu, v):
+    """Nodes whose first three kids are rejected for certain (tokens of probability 0) and whose fourth is a coin flip on
+    a token that each wave's first pass over the row writes: every wave must have read its probability by then. Tokens
+    and kids against the oracle, and nothing but the oracle's answer over repeated calls."""
+    n = 48
+    rng = np.random.default_rng(v)
+    p = rng.random((n, v)) ** 2
+    p[:, [3, 70, 150]] = 0.0
+    p /= p.sum(1, keepdims=True)
+    kids = []
+    for a in range(n):
+        x = int([0, 1, 63, 64, 100, 128, 190, 199][a % 8])
+        q = rng.random((3, v)) ** 2
+        q[:, x] = 0.0
+        q[:, [3, 70, 150]] += 0.1
+        q = q / q.sum(1, keepdims=True)
+        last = np.zeros(v)
+        last[x] = 2.0 * p[a, x]  # (the residuals so far only raise p[x]: accepted with probability a half or more)
+        last[(x + 1) % v] += 1.0 - last[x]
+        kids.append([(3, q[0]), (70, q[1]), (150, q[2]), (x, last if a % 3 else None), (3, q[0]), (x, q[1])])
+    pd = torch.from_numpy(p).to(gpu)
+    want = [spo.mss(p[a], kids[a], a, 9) for a in range(n)]
+    assert {r for _, r in want} >= {3, None}
+    for _ in range(3):
+        toks, ks = ge.spec.mss_batch(pd, kids, list(range(n)), [9] * n)
+        assert list(zip(toks, ks)) == want
+
+
 def test_rows_past_the_handles_size(ge, gpu):
     """A handle opened for one row of 64 tokens serves draw and mss over more rows of a longer vocabulary: its few
     slices widen and the rows go out in several launches."""
