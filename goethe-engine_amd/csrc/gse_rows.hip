@@ -110,20 +110,23 @@ __device__ __forceinline__ double row_total(const double *sums, int ns) {
   return t;
 }
 
-// The first j in [0, n) whose inclusive prefix before + sum(v(0..j)) reaches thr, 64 values at a time; before becomes
-// the prefix ahead of it. -1 when none does (before is then the whole sum).
+// The first j in [0, n) with v(j) > 0 whose inclusive prefix before + sum(v(0..j)) reaches thr, 64 values at a time; before
+// becomes the prefix ahead of it. -1 when none does. lastp: the last j seen with v(j) > 0 (-1 none). (A zero is never the
+// answer: the wave's scan adds in a tree, so a prefix may pass thr at a zero that follows the value that reached it.)
 template <typename VF>
-__device__ __forceinline__ int cross(int n, double thr, double &before, VF v) {
+__device__ __forceinline__ int cross(int n, double thr, double &before, int &lastp, VF v) {
+  lastp = -1;
   for (int j0 = 0; j0 < n; j0 += WAVE) {
     const int j = j0 + lane_id();
     const double x = j < n ? v(j) : 0.0;
     const double inc = before + wave_incl_scan_f64(x);
-    const uint64_t hit = ballot64(j < n && inc >= thr);
+    const uint64_t pos = ballot64(x > 0.0), hit = ballot64(x > 0.0 && inc >= thr);
     if (hit) {
       const int l = __builtin_ctzll(hit);
       before = l > 0 ? shfl_f64(inc, l - 1) : before;
       return j0 + l;
     }
+    if (pos) lastp = j0 + 63 - (int)__builtin_clzll(pos);
     before = shfl_f64(inc, WAVE - 1);
   }
   return -1;
@@ -131,8 +134,9 @@ __device__ __forceinline__ int cross(int n, double thr, double &before, VF v) {
 
 // draw() of a row whose slices have been summed (by one wave; every lane gets it): the first token whose inclusive
 // prefix reaches u * total, at most the last token with a positive weight; -1 when no weight is positive. A total that
-// is NaN gives the first token (count(c < NaN) = 0). A prefix of tokens may round below the slice's own sum: the draw
-// then takes the crossing segment's (or slice's) last token.
+// is NaN gives the first token (count(c < NaN) = 0), and so does u = 0; any other token has a positive weight. The sums of
+// slices, segments and tokens round apart, so a slice's segments, or a segment's tokens, may stay below what the sum
+// above them reached: the draw then takes the last of them with a positive weight.
 template <typename EW>
 __device__ __forceinline__ int row_draw(const RowSlices &rs, int V, double u, double total, const double *sums,
                                         const double *segs, const int32_t *lasts, EW ev) {
@@ -141,17 +145,17 @@ __device__ __forceinline__ int row_draw(const RowSlices &rs, int V, double u, do
   lst = (int)wave_max_u32((uint32_t)(lst + 1)) - 1;
   if (lst < 0) return -1;
   const double thr = u * total;
-  if (thr != thr) return 0;
+  if (!(thr > 0.0)) return 0;
   double before = 0.0;
-  const int sx = cross(rs.ns, thr, before, [&](int j) { return ld_ag(&sums[j]); });
+  int lp;
+  const int sx = cross(rs.ns, thr, before, lp, [&](int j) { return ld_ag(&sums[j]); });
   if (sx < 0) return lst;
   const double *sg = segs + (size_t)sx * RSEG;
-  const int g = cross(RSEG, thr, before, [&](int j) { return ld_ag(&sg[j]); });
-  const int s1 = (sx + 1) * RS * rs.sub;
-  if (g < 0) return min(min(s1, V) - 1, lst);
+  const int g = cross(RSEG, thr, before, lp, [&](int j) { return ld_ag(&sg[j]); });
+  if (g < 0) return ld_ag(&lasts[sx]);
   const int t0 = (sx * RSEG + g) * WAVE * rs.sub, t1 = min(t0 + WAVE * rs.sub, V);
-  const int k = cross(t1 - t0, thr, before, [&](int j) { return ev(t0 + j); });
-  return min(k < 0 ? t1 - 1 : t0 + k, lst);
+  const int k = cross(t1 - t0, thr, before, lp, [&](int j) { return ev(t0 + j); });
+  return t0 + (k < 0 ? lp : k);
 }
 
 struct DrawArgs {
@@ -616,11 +620,13 @@ __device__ __forceinline__ void pick_draw(const PickArgs &a, int row, int kd, co
     last = (int)wave_max_u32((uint32_t)(last + 1)) - 1;
     const double thr = uniform64(mix64(a.b.seed[row], SALT_DRAFT + (uint64_t)kd), a.b.at[row]) * E;
     double before = 0.0;
-    const int sx = cross(a.ns, thr, before, weight);
-    tok = last;
-    if (sx >= 0) {
+    int lp;
+    const int sx = cross(a.ns, thr, before, lp, weight);
+    tok = thr > 0.0 ? last : 0;  // (u = 0 draws the first token, whatever its mass)
+    if (thr > 0.0 && sx >= 0) {
       const double m = ld_ag(&mx[sx]), sc = exp_nonpos(m - M, etab);
-      const double ts = sc > 0.0 ? (thr - before) / sc : 0.0;  // the threshold in the slice's own masses
+      // the threshold in the slice's own masses (positive: a token of mass 0 never reaches it)
+      const double ts = fmax((thr - before) / sc, 0x1p-1000);
       const Fx *sg = a.seg + (o + sx) * (RSEG / 2);
       Fx f = lane < L::NSEG ? Fx{ld_ag(&sg[lane].hi), ld_ag(&sg[lane].lo)} : Fx{0, 0};
       Fx inc{wave_incl_scan_u64(f.hi), wave_incl_scan_u64(f.lo)};

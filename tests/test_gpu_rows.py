@@ -33,6 +33,31 @@ def test_draw_sizes(ge, gpu, v):
         ge.sampling.draw(torch.zeros(v, dtype=torch.float64, device=gpu), 0.5)
 
 
+def test_draw_never_takes_a_zero(ge, gpu):
+    """Rows with long runs of zeros, u at the prefix of a random token and the doubles next to it: the slices, segments
+    and tokens are summed in different orders, and whichever of them rounds to the threshold first, the drawn token has
+    a positive weight and its exact prefix lies within rounding of u (sums of 9001 terms: 1e-13)."""
+    lib = ge._lib
+    v, rows = 9001, 6000
+    rng = np.random.default_rng(12)
+    q = rng.random((20, v)) * (rng.random((20, v)) < 0.02)
+    q[:, 4090:4200] = 0.0
+    c = q.cumsum(1)
+    src = np.arange(rows) % 20
+    at = np.array([rng.choice(np.nonzero(q[r])[0]) for r in src])
+    u = c[src, at] / c[src, -1] + rng.integers(-6, 7, rows) * 2.0 ** -53
+    u = np.clip(u, 2.0 ** -53, 1.0 - 2.0 ** -53)
+    qd = torch.from_numpy(q).to(gpu)[torch.from_numpy(src).to(gpu)].contiguous()
+    ud = torch.from_numpy(u).to(gpu)
+    out = torch.full((rows,), -7, dtype=torch.int32, device=gpu)
+    h = lib.handle(gpu.index, 64, v)
+    h.call("gse_draw", qd.data_ptr(), v, rows, v, ud.data_ptr(), out.data_ptr(), lib.stream_of(gpu.index))
+    t = out.cpu().numpy()
+    assert (t >= 0).all() and (q[src, t] > 0).all(), t[q[src, t] <= 0]
+    lo, hi = (c[src, t] - q[src, t]) / c[src, -1], c[src, t] / c[src, -1]
+    assert (u >= lo - 1e-13).all() and (u <= hi + 1e-13).all()
+
+
 def _nodes(v, n, rng):
     """Nodes of 0 .. 5 kids over [n, v] targets: kids with a distribution of their own, kids sharing one, one-hot kids;
     the kids' tokens are where q most exceeds p, so that most are rejected and the deeper levels run."""
