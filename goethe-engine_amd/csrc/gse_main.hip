@@ -247,8 +247,8 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
     // prefixes. c_last is at least the prefix of the first rank that may fail, or, past the head, the head's mass and
     // (top-p the only cut) top_p S; at most the prefix of the first that surely fails, or top_p S and one element more
     // (the last kept one, at most the head's last), or S. Only a token is wanted: dist and verify nodes that take
-    // dist + mss need the boundary itself.
-    if (n == 0 || a.mode != MODE_SAMPLE || (a.tree && (P.flags & GSE_ROW_MSS)) || htot < HEAD_DRAW * topp * Sm)
+    // dist + mss need the boundary itself. (m1 = 0: the bound exceeds S, so even rank 0 may fail, and no prefix comes before)
+    if (n == 0 || m1 == 0 || a.mode != MODE_SAMPLE || (a.tree && (P.flags & GSE_ROW_MSS)) || htot < HEAD_DRAW * topp * Sm)
       return EV_HARD;
     const double clo = m1 != NONE ? ee[m1 - 1] : P.top_k > 0 || minp > 0.0 ? htot : fmax(htot, tlo);
     const double chi = m2 != NONE ? ee[m2 - 1] : fmin(Sm + B, thi + (n > 1 ? ee[n - 1] - ee[n - 2] : htot));

@@ -93,6 +93,19 @@ def test_draws_settled_in_the_head(ge, gpu, dtype):
         assert main >= (4 if n == 1 else n // 2), (n, main)
 
 
+@pytest.mark.parametrize("parts", [6, 16])
+def test_bound_past_the_sum(ge, gpu, parts):
+    """Logits of 2^27 (a ulp apart: 8) make the bound on the unlisted mass (1.8e-7 |z| relative) larger than the whole
+    sum: the head cannot even tell that its first rank is kept, and the split-row pass decides."""
+    v = parts * 8192
+    x = np.full((4, v), 2.0 ** 27 - 8, np.float32)
+    for p in range(parts):  # (40 lanes of every part's sample hold a maximum: the parts list these and no more)
+        x[:, p * 8192:p * 8192 + 2048:50] = 2.0 ** 27
+    P = ge.sampling.SamplingParams
+    paths = _check(ge, gpu, x, [P(temperature=1.0, top_p=[0.5, 0.8, 0.3, 0.7][r]) for r in range(4)], 5)
+    assert (paths == ge._lib.PATH_DEEP).any()
+
+
 def test_masked_rows_whose_samples_are_empty(ge, gpu):
     """Masked rows whose allowed runs lie outside most parts' samples (those parts start listing everything). Greedy rows
     with logprobs, sampled rows with and without, T = 1 and not: tokens, ids and logprobs against the oracle, none on the
