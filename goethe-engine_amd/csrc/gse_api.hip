@@ -548,6 +548,7 @@ GSE_API int gse_qprob(gse_handle *h, const gse_qrows *qrows, uint32_t vocab, dou
   if (!q.q || !q.temperature || !out) return fail(h, GSE_E_ARG, "q, temperature and out are required");
   if (vocab == 0 || q.ld < (int64_t)vocab || out_ld < (int64_t)vocab)
     return fail(h, GSE_E_ARG, "vocab 0, q ld < vocab or out_ld < vocab");
+  if (vocab > (uint32_t)INT32_MAX) return fail(h, GSE_E_ARG, "vocab %u past 2^31 - 1", vocab);
   DeviceGuard g(h->device);
   hipError_t e = gse::launch_qprob(rows_ws(h), q, (int)vocab, out, out_ld, (hipStream_t)stream);
   return e == hipSuccess ? GSE_OK : hip_fail(h, e, "qprob launch");
@@ -558,6 +559,7 @@ GSE_API int gse_draw(gse_handle *h, const double *q, int64_t q_ld, uint32_t rows
   if (!h) return fail(nullptr, GSE_E_ARG, "null handle");
   if (!q || !u || !out) return fail(h, GSE_E_ARG, "q, u and out are required");
   if (vocab == 0 || q_ld < (int64_t)vocab) return fail(h, GSE_E_ARG, "vocab 0 or q_ld < vocab");
+  if (vocab > (uint32_t)INT32_MAX) return fail(h, GSE_E_ARG, "vocab %u past 2^31 - 1", vocab);
   if (rows == 0) return GSE_OK;
   DeviceGuard g(h->device);
   hipError_t e = gse::launch_draw(rows_ws(h), q, q_ld, (int)rows, (int)vocab, u, out, (hipStream_t)stream);
@@ -572,6 +574,7 @@ GSE_API int gse_mss(gse_handle *h, const gse_mss_batch *in) {
     return fail(h, GSE_E_ARG, "p, kid_tok, kid_q, seed, idx, out_token, out_kid are required");
   if (b.vocab == 0 || b.p_ld < (int64_t)b.vocab) return fail(h, GSE_E_ARG, "vocab 0 or p_ld < vocab");
   if (b.q && b.q_ld < (int64_t)b.vocab) return fail(h, GSE_E_ARG, "q_ld < vocab");
+  if (b.vocab > (uint32_t)INT32_MAX) return fail(h, GSE_E_ARG, "vocab %u past 2^31 - 1", b.vocab);
   if (b.nodes == 0) return GSE_OK;
   DeviceGuard g(h->device);
   hipError_t e = gse::launch_mss(rows_ws(h), b, (hipStream_t)b.stream);

@@ -50,7 +50,8 @@ template <typename LD, typename EV>
 __device__ __forceinline__ void slice_sum(const RowSlices &rs, int s, int V, LD load, EV ev, double *segs, double *sum,
                                           int32_t *last, RowsShared &sh) {
   const int lane = lane_id(), w = threadIdx.x >> 6;
-  const int s0 = s * RS * rs.sub;
+  // (unsigned: past the end of a row of nearly 2^31 tokens)
+  const uint32_t s0 = (uint32_t)(s * RS * rs.sub), end = (uint32_t)V;
   int lst = -1;
   if (rs.sub == 1) {
     // eight segments' loads in flight at a time
@@ -58,12 +59,13 @@ __device__ __forceinline__ void slice_sum(const RowSlices &rs, int s, int V, LD 
     for (int h = 0; h < RGS; h += 8) {
       decltype(load(0)) r[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) r[k] = load(min(s0 + ((h + k) * RW + w) * WAVE + lane, V - 1));
+      for (int k = 0; k < 8; ++k) r[k] = load((int)min(s0 + (uint32_t)(((h + k) * RW + w) * WAVE + lane), end - 1u));
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const int g = (h + k) * RW + w, t = s0 + g * WAVE + lane;
-        const double v = t < V ? ev(t, r[k]) : 0.0;
-        if (v > 0.0) lst = t;
+        const int g = (h + k) * RW + w;
+        const uint32_t t = s0 + (uint32_t)(g * WAVE + lane);
+        const double v = t < end ? ev((int)t, r[k]) : 0.0;
+        if (v > 0.0) lst = (int)t;
         const double sg = wave_sum_f64(v);
         if (lane == 0) sh.seg[g] = sg;
       }
@@ -74,9 +76,9 @@ __device__ __forceinline__ void slice_sum(const RowSlices &rs, int s, int V, LD 
       const int g = q * RW + w;
       double sg = 0.0;
       for (int c = 0; c < rs.sub; ++c) {
-        const int t = s0 + (g * rs.sub + c) * WAVE + lane;
-        const double v = t < V ? ev(t, load(t)) : 0.0;
-        if (v > 0.0) lst = t;
+        const uint32_t t = s0 + (uint32_t)((g * rs.sub + c) * WAVE + lane);
+        const double v = t < end ? ev((int)t, load((int)t)) : 0.0;
+        if (v > 0.0) lst = (int)t;
         sg += wave_sum_f64(v);
       }
       if (lane == 0) sh.seg[g] = sg;
@@ -153,8 +155,8 @@ __device__ __forceinline__ int row_draw(const RowSlices &rs, int V, double u, do
   const double *sg = segs + (size_t)sx * RSEG;
   const int g = cross(RSEG, thr, before, lp, [&](int j) { return ld_ag(&sg[j]); });
   if (g < 0) return ld_ag(&lasts[sx]);
-  const int t0 = (sx * RSEG + g) * WAVE * rs.sub, t1 = min(t0 + WAVE * rs.sub, V);
-  const int k = cross(t1 - t0, thr, before, lp, [&](int j) { return ev(t0 + j); });
+  const int t0 = (sx * RSEG + g) * WAVE * rs.sub, nt = min(WAVE * rs.sub, V - t0);
+  const int k = cross(nt, thr, before, lp, [&](int j) { return ev(t0 + j); });
   return t0 + (k < 0 ? lp : k);
 }
 
@@ -280,7 +282,7 @@ __device__ __noinline__ void mss_rest(const MssArgs &a, int node, MssKid k, Rows
     }
     __syncthreads();  // every thread has read p[x] before it changes
     double s = 0.0;
-    for (int t = tid; t < V; t += RT) {
+    for (uint32_t t = tid; t < (uint32_t)V; t += RT) {
       const double v = residual(p[t], k, k.q ? k.q[t] : 0.0, t);
       p[t] = v;
       s += v;
@@ -291,7 +293,7 @@ __device__ __noinline__ void mss_rest(const MssArgs &a, int node, MssKid k, Rows
     double tot = 0.0;
     for (int w = 0; w < RW; ++w) tot += sh.red[w];
     if (tot > 0.0)
-      for (int t = tid; t < V; t += RT) p[t] = p[t] / tot;
+      for (uint32_t t = tid; t < (uint32_t)V; t += RT) p[t] = p[t] / tot;
     __syncthreads();
     k = kid_from(b, node, k.r + 1);
   }
@@ -376,7 +378,7 @@ __global__ __launch_bounds__(RT) void mss_kernel(MssArgs a) {
       }
     } else {
       __syncthreads();  // (every wave has read p[kn.x], which the loop writes)
-      for (int t = tid; t < V; t += RT) {
+      for (uint32_t t = tid; t < (uint32_t)V; t += RT) {
         const double v = at(t);
         p[t] = total > 0.0 ? v / total : v;
       }
@@ -401,9 +403,9 @@ struct RLay {
 };
 
 template <int DT, bool AL>
-__device__ __forceinline__ void load_vec(const char *base, int t0, int V, float *x) {
-  using L = RLay<DT>;
-  if (AL && t0 + L::VEC <= V) {
+__device__ __forceinline__ void load_vec(const char *base, uint32_t t0, int V, float *x) {
+  using L = RLay<DT>;  // (t0 unsigned: it may lie past the end of a row of nearly 2^31 tokens)
+  if (AL && t0 + L::VEC <= (uint32_t)V) {
     if constexpr (DT == GSE_BF16) {
       const uint4 u = *reinterpret_cast<const uint4 *>(base + (size_t)t0 * 2);
       const uint32_t w[4] = {u.x, u.y, u.z, u.w};
@@ -422,11 +424,11 @@ __device__ __forceinline__ void load_vec(const char *base, int t0, int V, float 
   } else {
 #pragma unroll
     for (int e = 0; e < L::VEC; ++e) {
-      const int t = min(t0 + e, V - 1);
+      const uint32_t t = min(t0 + e, (uint32_t)V - 1u);
       float f;
       if constexpr (DT == GSE_BF16) f = bf16_to_f32(((const uint16_t *)base)[t]);
       else f = ((const float *)base)[t];
-      x[e] = t0 + e < V ? f : -INFINITY;
+      x[e] = t0 + e < (uint32_t)V ? f : -INFINITY;
     }
   }
 }
@@ -811,8 +813,8 @@ __global__ __launch_bounds__(RT) void qstats_kernel(QprobArgs a) {
   if (tid < 64) sh.etab[tid] = EXP2_64[tid];
   double M = -INFINITY, E = 0.0;
   for (int c = 0; c < a.rs.sub; ++c) {  // (one slice, unless the workspace's slices widen)
-    const int s0 = (s * a.rs.sub + c) * RS;
-    if (s0 >= a.V) break;
+    const uint32_t s0 = (uint32_t)(s * a.rs.sub + c) * RS;
+    if (s0 >= (uint32_t)a.V) break;
     float x[RE], xm = -INFINITY;
     bool nan = false;
 #pragma unroll
@@ -899,8 +901,8 @@ __global__ __launch_bounds__(RT) void qprob_kernel(QprobArgs a) {
   }
   // (the slice's loads overlap the row's sums)
   for (int c = 0; c < a.rs.sub; ++c) {
-    const int s0 = (s * a.rs.sub + c) * RS;
-    if (s0 >= a.V) break;
+    const uint32_t s0 = (uint32_t)(s * a.rs.sub + c) * RS;
+    if (s0 >= (uint32_t)a.V) break;
     float x[RE];
 #pragma unroll
     for (int v = 0; v < L::NV; ++v) load_vec<DT, AL>(base, s0 + (v * RT + tid) * L::VEC, a.V, &x[v * L::VEC]);
@@ -908,11 +910,11 @@ __global__ __launch_bounds__(RT) void qprob_kernel(QprobArgs a) {
     const double M = sh.M, E = sh.E;
 #pragma unroll
     for (int v = 0; v < L::NV; ++v) {
-      const int t0 = s0 + (v * RT + tid) * L::VEC;
+      const uint32_t t0 = s0 + (v * RT + tid) * L::VEC;
 #pragma unroll
       for (int e = 0; e < L::VEC; ++e) {
         const double q = M != M ? M : exp_nonpos((double)x[v * L::VEC + e] / t - M, sh.etab) / E;
-        if (t0 + e < a.V) o[t0 + e] = q;
+        if (t0 + e < (uint32_t)a.V) o[t0 + e] = q;
       }
     }
   }
@@ -921,7 +923,7 @@ __global__ __launch_bounds__(RT) void qprob_kernel(QprobArgs a) {
 // The slicing of rows of V tokens, and the rows that one launch takes (at least 1) of the workspace's R rows of S slices.
 RowSlices slices_of(const RowsWs &w, int V, int *rows) {
   const int64_t cap = (int64_t)w.rows * w.slices;
-  int64_t ns = (V + RS - 1) / RS, sub = 1;
+  int64_t ns = ((int64_t)V + RS - 1) / RS, sub = 1;
   if (ns > cap) {
     sub = (ns + cap - 1) / cap;
     ns = (V + RS * sub - 1) / (RS * sub);

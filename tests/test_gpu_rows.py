@@ -164,6 +164,42 @@ def test_rows_past_the_handles_size(ge, gpu):
     h.close()
 
 
+def test_rows_of_nearly_2_31_tokens(ge, gpu):
+    """The last slice of a row of 2^31 - 1 tokens reaches past 2^31: draw and qprob read and write inside the row, and a
+    longer row is refused."""
+    lib = ge._lib
+    v = 2 ** 31 - 1
+    q = torch.zeros(v, dtype=torch.float64, device=gpu)
+    q[5] = q[v - 1] = 1.0
+    h = lib.Handle(gpu.index, 64, 64)
+    st = lib.stream_of(gpu.index)
+    out = torch.zeros(1, dtype=torch.int32, device=gpu)
+    for u, want in ((0.3, 5), (0.7, v - 1)):
+        ut = torch.tensor([u], dtype=torch.float64, device=gpu)
+        h.call("gse_draw", q.data_ptr(), v, 1, v, ut.data_ptr(), out.data_ptr(), st)
+        assert out.item() == want
+    x = torch.full((1, v), -float("inf"), dtype=torch.bfloat16, device=gpu)
+    x[0, 3] = x[0, v - 1] = 2.0
+    t = torch.ones(1, dtype=torch.float64, device=gpu)
+    r = lib.QRows()
+    r.size, r.kind = C.sizeof(lib.QRows), lib.Q_LOGITS_BF16
+    r.rows, r.q, r.ld, r.temperature = 1, x.data_ptr(), v, t.data_ptr()
+    h.call("gse_qprob", C.byref(r), v, q.data_ptr(), v, st)
+    assert q[3].item() == 0.5 and q[v - 1].item() == 0.5 and torch.count_nonzero(q).item() == 2
+    with pytest.raises(RuntimeError, match="2\\^31"):
+        h.call("gse_draw", q.data_ptr(), v + 1, 1, v + 1, t.data_ptr(), out.data_ptr(), st)
+    r.ld = v + 1
+    with pytest.raises(RuntimeError, match="2\\^31"):
+        h.call("gse_qprob", C.byref(r), v + 1, q.data_ptr(), v + 1, st)
+    m = lib.MssBatch()
+    m.size, m.nodes, m.vocab, m.max_kids = C.sizeof(lib.MssBatch), 1, v + 1, 1
+    m.p, m.p_ld = q.data_ptr(), v + 1
+    m.kid_tok = m.kid_q = m.seed = m.idx = m.out_token = m.out_kid = out.data_ptr()
+    with pytest.raises(RuntimeError, match="2\\^31"):
+        h.call("gse_mss", C.byref(m))
+    h.close()
+
+
 def _pick_rows(v, rng):
     """Rows with ties everywhere (one value; two values), with the best tokens side by side, with -inf in most places,
     with a single finite token, and plain ones."""
