@@ -268,49 +268,48 @@ __device__ __forceinline__ MssTok<D> mss_load(const double *p, const MssKid (&k)
   return m;
 }
 
-// The kids past level MSS_LEVELS, by one workgroup, in place in p (p: the distribution before kid k's test, written by
-// this workgroup): the draw's sums are left in the node's workspace.
-__device__ __noinline__ void mss_rest(const MssArgs &a, int node, MssKid k, RowsShared &sh) {
+// The kids past level MSS_LEVELS, by one workgroup, in place in p: the residual of the level before (written by this
+// workgroup), total its sum. A kid is one pass over the row: the division by the sum before, the residual, and the slices'
+// sums, which the next test and the draw use (a residual that is not divided draws the same), with 16 tokens a thread in
+// flight. Bound by the chain of one workgroup's slices. Every kid rejected, us a call:
+//   16 nodes of 128256: 4 kids 517, 16 kids 3070 (two passes a kid of 256 tokens at a time and a third for the draw: 819,
+//   5700; one workgroup of 1024 threads a node over contiguous runs: 1823, 6790)
+//   64 nodes of 151936: 4 kids 1240, 16 kids 8110, one-hot 850, 5150 (1840, 13400, 1410, 8720; 3380, 12600, 2700, 9860)
+__device__ __noinline__ void mss_rest(const MssArgs &a, int node, MssKid k, double total, RowsShared &sh) {
   const gse_mss_batch &b = a.b;
   const int V = (int)b.vocab, tid = threadIdx.x;
   double *p = b.p + (int64_t)node * b.p_ld;
-  while (k.r >= 0) {
+  const size_t o = (size_t)(node - a.node0) * a.rs.ns;
+  for (;;) {
+    __syncthreads();  // (p is written)
     const double px = p[k.x];
-    if (mss_accepts(b, node, k, px)) {
+    if (mss_accepts(b, node, k, total > 0.0 ? px / total : px)) {
       if (tid == 0) mss_out(b, node, k.x, k.r);
       return;
     }
     __syncthreads();  // every thread has read p[x] before it changes
-    double s = 0.0;
-    for (uint32_t t = tid; t < (uint32_t)V; t += RT) {
-      const double v = residual(p[t], k, k.q ? k.q[t] : 0.0, t);
-      p[t] = v;
-      s += v;
+    const double *q = k.q ? k.q : p;  // (one-hot: a load that is dropped)
+    for (int s = 0; s < a.rs.ns; ++s) {
+      slice_sum(a.rs, s, V, [&](int t) { return MssTok<1>{p[t], {q[t]}}; },
+                [&](int t, const MssTok<1> &m) {
+                  return p[t] = residual(total > 0.0 ? m.p / total : m.p, k, m.q[0], t);
+                },
+                a.seg + (o + s) * RSEG, a.sum + o + s, a.last + o + s, sh);
     }
-    s = wave_sum_f64(s);
-    if (lane_id() == 0) sh.red[tid >> 6] = s;
-    __syncthreads();
-    double tot = 0.0;
-    for (int w = 0; w < RW; ++w) tot += sh.red[w];
-    if (tot > 0.0)
-      for (uint32_t t = tid; t < (uint32_t)V; t += RT) p[t] = p[t] / tot;
-    __syncthreads();
+    total = row_total(a.sum + o, a.rs.ns);
     k = kid_from(b, node, k.r + 1);
-  }
-  const size_t o = (size_t)(node - a.node0) * a.rs.ns;
-  for (int s = 0; s < a.rs.ns; ++s) {
-    slice_sum(a.rs, s, V, [&](int t) { return p[t]; }, [](int, double v) { return v; }, a.seg + (o + s) * RSEG,
-              a.sum + o + s, a.last + o + s, sh);
+    if (k.r < 0) break;
   }
   if (tid >= WAVE) return;
-  const double total = row_total(a.sum + o, a.rs.ns);
   const int j = row_draw(a.rs, V, uniform64(mix64(b.seed[node], SALT_RES), b.idx[node]), total, a.sum + o,
                          a.seg + o * RSEG, a.last + o, [&](int t) { return p[t]; });
   if (tid == 0) mss_out(b, node, j, -1);
 }
 
+// (at least three waves per SIMD: without the bound mss_rest's registers leave two, and 64 nodes of 151936 with three kids
+// rejected take 137 us instead of 128)
 template <int D>
-__global__ __launch_bounds__(RT) void mss_kernel(MssArgs a) {
+__global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(3, 8))) void mss_kernel(MssArgs a) {
   __shared__ RowsShared sh;
   const gse_mss_batch &b = a.b;
   const int s = blockIdx.x, n = blockIdx.y, node = a.node0 + n, tid = threadIdx.x;
@@ -378,12 +377,17 @@ __global__ __launch_bounds__(RT) void mss_kernel(MssArgs a) {
       }
     } else {
       __syncthreads();  // (every wave has read p[kn.x], which the loop writes)
-      for (uint32_t t = tid; t < (uint32_t)V; t += RT) {
-        const double v = at(t);
-        p[t] = total > 0.0 ? v / total : v;
+      for (uint32_t t0 = 0; t0 < (uint32_t)V; t0 += 4 * RT) {
+        MssTok<D> m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = mss_load<D>(p, k, (int)min(t0 + i * RT + tid, (uint32_t)V - 1u));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t t = t0 + i * RT + tid;
+          if (t < (uint32_t)V) p[t] = level<D>(k, sig, m[i].p, m[i].q, (int)t);
+        }
       }
-      __syncthreads();
-      mss_rest(a, node, kn, sh);  // (tests kid kn once more: the same answer)
+      mss_rest(a, node, kn, total, sh);  // (tests kid kn once more: the same answer)
     }
     return;
   }
