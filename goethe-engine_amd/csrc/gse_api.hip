@@ -199,6 +199,8 @@ gse::ScanArgs make_args(gse_handle *h, const gse_batch &b, int mode) {
   a.kt = a.plen > gse::PTOK ? (int)(((int64_t)gse::KT * a.plen + gse::PTOK - 1) / gse::PTOK)
                             : plain ? gse::KT : gse::KT_HM;
   const bool many = a.nparts > gse::KT_PARTS;  // (rows of many parts share out the listing targets)
+  a.kown = std::min(2 * a.kt, gse::KT_OWN / a.nparts);
+  a.klane = many ? (a.plen + 2047) / 2048 : 0;
   if (many) a.kt = std::max(gse::KT_MIN, a.kt * gse::KT_SHARE / a.nparts);
   a.kshare = 256 * std::min((many ? gse::KT_SHARE : gse::KT_TOPK), a.nparts) / a.nparts;
   a.kmin = many ? gse::KT_MIN : gse::KT_MINK;

@@ -65,6 +65,15 @@ constexpr int KT_MIN = 24;    // resolve gathers and which overflow its head (20
 // 4 parts: 98.3, 97.5, 97.5 us; the same share with 16 parts and 48 cost 4 rows 28.1 -> 32.8 us.
 constexpr int KT_TOPK = 2;
 constexpr int KT_MINK = 48;
+// What a row needs by rank may all lie in one part. A top-k row's target is at least top_k + 8 where that is at most twice
+// the parts' target; a row's with nlp logprobs (a head of fewer needs the exact path) at least 3/2 nlp + 8 and, in rows of
+// more than KT_PARTS parts, nlp / 4 + 2 of the sample's lane maxima (in ids ordered by rank a lane holds four best tokens in
+// a row), but at most KT_OWN over the parts: the head, the lists' entries above the highest of the parts' thresholds, then
+// holds 1300 to 1900 of its 2048 entries in rows of 16 to 32 parts without such order (past 2048 those need the exact
+// path). Logits falling with the token id: one row of 128256 with 64 logprobs 2577 -> 34 us (greedy 336 -> 26), 16 rows with
+// top-k 40 53 -> 28 us; in random order 25.1 -> 33.5, 24.1 -> 31.5 and 24.9 -> 27.3 us (with unshared targets 1795, 302
+// and 36).
+constexpr int KT_OWN = 2304;
 constexpr int KT_VALVE = 222; // the listing target at which a part's first-chunk valve is CAPW / 4 (scaled with kt)
 constexpr int PCHUNK = 1024;  // part lengths are multiples of this (one wave chunk)
 constexpr int PMIN = 8192;    // tokens per part, at least, when a small batch is split to fill the device: every part
@@ -150,6 +159,7 @@ struct ScanArgs {
   int dtype, V, rows, nch, mode, force_exact, xcd_map;
   int nparts, plen;  // the main pass: parts per row, tokens per part (a multiple of 1024; the last part may be shorter)
   int kshare, kmin;  // rows with top-k: a part's share of 2 top_k + 32 in 1/256, and its least target
+  int kown, klane;   // the largest target that a row's logprobs raise a part to; a lane maximum's share of it
   int kt, vfirst;    // tokens of a part its listing threshold aims to leave above it; list length that first opens the valve
   int pmajor;        // workgroup L streams part L / rows8 of row L % rows8 (else the parts of a row are consecutive)
   const gse_row *params;

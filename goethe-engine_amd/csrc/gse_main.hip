@@ -1211,7 +1211,8 @@ __device__ __forceinline__ bool part_body(const ScanArgs &a, const gse_row &P, c
     // sample). kp is scaled so that about T tokens of the part lie above it: kp = T * (allowed tokens in the sample) /
     // (allowed tokens in the part), counted exactly, so that a mask whose allowed tokens cluster in runs does not skew
     // it. T = a.kt (200 for a part of at most PTOK tokens, 150 in a call with histories or masks, less for rows of many
-    // parts), or a share of 2 top_k + 32 (at most 2 a.kt) for rows that keep at most top_k elements.
+    // parts), or a share of 2 top_k + 32 (at most 2 a.kt) for rows that keep at most top_k elements; at least what a row
+    // needs of its top ranks.
     uint32_t as = 0;
 #pragma unroll
     for (int i = 0; i < EPL; ++i) as += x0[i] > -INFINITY ? 1u : 0u;
@@ -1232,8 +1233,16 @@ __device__ __forceinline__ bool part_body(const ScanArgs &a, const gse_row &P, c
       Ap += sh.wflags[q];
     }
     const uint32_t kt = (uint32_t)a.kt;
-    const uint32_t tk = (uint32_t)(2 * max(min(P.top_k, 4096), nlp_of(a, P)) + 32) * (uint32_t)a.kshare >> 8;
-    const uint32_t T = P.top_k > 0 ? min(2u * kt, max(tk, (uint32_t)a.kmin)) : kt;
+    // A part may hold every token that a row needs by its rank (ids ordered by frequency, a grammar's one run): the top-k
+    // tokens, where twice the target has room for them, and the logprobs' (KT_OWN).
+    const uint32_t K = (uint32_t)min(P.top_k, 4096);  // (when > 0)
+    const uint32_t tk = max((2u * K + 32u) * (uint32_t)a.kshare >> 8, K + 8u <= 2u * kt ? K + 8u : 0u);
+    uint32_t T = P.top_k > 0 ? min(2u * kt, max(tk, (uint32_t)a.kmin)) : kt;
+    const int nlp = nlp_of(a, P), own = nlp > 0 ? min(max(3 * nlp / 2 + 8, (nlp / 4 + 2) * a.klane), a.kown) : 0;
+    if (own > (int)T) {
+      T = (uint32_t)own;
+      rn.vnext = max(rn.vnext, (uint32_t)(CAPW / 4) * T / (uint32_t)KT_VALVE + 1u);
+    }
     // (a sample with few allowed tokens estimates nothing: then the lowest lane maximum, and the valve bounds the lists)
     const uint32_t kp = As < 16u ? max(act, 1u) : max(1u, min(act, (T * As + Ap - 1) / max(Ap, 1u)));  // (T As < 2^22)
     uint32_t r = 0;

@@ -93,6 +93,42 @@ def test_draws_settled_in_the_head(ge, gpu, dtype):
         assert main >= (4 if n == 1 else n // 2), (n, main)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n,v,order", [(n, v, o) for n, v in [(1, 128256), (4, 131072), (2, 262144), (8, 32000), (1, 9000)]
+                                       for o in ("falling", "none")] + [(4, 131072, "one part")])
+def test_best_tokens_in_one_part(ge, gpu, n, v, dtype, order):
+    """Rows whose ids are ordered by rank, or whose best tokens fill one part of the main pass: greedy and nucleus rows
+    with 20 and 64 logprobs and top-k rows need no exact path, and the ordered top-k rows end in the main pass (a part in
+    any order lists within a fifth of its target, 48 here: some rows fall short of their 40)."""
+    rng = np.random.default_rng(v + n)
+    x = _zipf(rng, n, v)
+    x -= x.mean(axis=1, keepdims=True)  # (ordered parts span little: near 0 their values stay apart in 16 key bits)
+    if order != "none":
+        x = -np.sort(-x, axis=1)
+    if order == "one part":  # (part 8 of 16, in any order)
+        x = np.concatenate([rng.permuted(x[:, 8192:v // 2 + 8192], axis=1), rng.permuted(x[:, :8192], axis=1),
+                            x[:, v // 2 + 8192:]], axis=1)
+    x = torch.from_numpy(x)
+    x = x.bfloat16() if dtype == "bf16" else x
+    x32, xd = x.float().numpy(), x.to(gpu)
+    P = ge.sampling.SamplingParams
+    u = rng.random(n)
+    for p in (P(logprobs=20), P(logprobs=64), P(temperature=0.9, top_p=0.9, logprobs=20),
+              P(temperature=0.9, top_p=0.9, logprobs=64), P(temperature=0.8, top_k=40, top_p=0.95),
+              P(temperature=0.8, top_k=40)):
+        sel = ge.sampling.sample_ex(xd, [p] * n, None, None, None, uniforms=u)
+        paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
+        want = ora.sample_full(x32, [p] * n, None, None, None, None, u)
+        assert sel.tolist() == [w["token"] for w in want], p
+        assert (paths == ge._lib.PATH_EXACT).sum() == 0, (p, paths)
+        if p.top_k and order != "one part":
+            assert (paths == ge._lib.PATH_MAIN).all(), (p, paths)
+        if p.logprobs:
+            ids = sel.logprob_ids.cpu().numpy()
+            for r in range(n):
+                assert list(ids[r, :p.logprobs]) == list(want[r]["logprob_ids"]), p
+
+
 @pytest.mark.parametrize("parts", [6, 16])
 def test_bound_past_the_sum(ge, gpu, parts):
     """Logits of 2^27 (a ulp apart: 8) make the bound on the unlisted mass (1.8e-7 |z| relative) larger than the whole
