@@ -5,9 +5,9 @@
 // with integer atomics (the same sums in any order), and the last slice of a row to finish a phase (atomic ticket)
 // carries on with the row. Every workgroup runs all its count items before any pick item.
 //
-//   count:  each slice recomputes z exactly as the main pass does and adds a 512-bin histogram of
+//   count:  each slice recomputes z exactly as the main pass does and adds a histogram (DNB bins) of
 //           d = z_max - z: counts and exact fixed-point masses (fp64 exp, whole multiples of 2^-40 and 2^-64; bins
-//           1/32 wide, wider past d = 12, the last one open). d is monotone in z, so the bins follow the stable order and ties share
+//           1/32 wide, wider past d = 16, the last one open). d is monotone in z, so the bins follow the stable order and ties share
 //           a bin. The row's last slice plans: the bins that hold the last kept element (top-p, top-k and min-p cuts)
 //           and the bins that may hold the draw, whether they hold at most DCAP elements, and the exact masses of the
 //           regions before and between them; then it publishes the plan's status.
@@ -29,14 +29,16 @@ namespace {
 
 using namespace strm;
 
-// Histogram bins of d = z_max - z: 1/32 wide to d = 12 (bin 384), 1/8 wide to d = 20 (bin 448), then 1/2 wide; the last one
-// (from d = 51.5) is open. Most rows' cuts lie in the fine bins; the wide ones spread the tail of a row whose logits range
-// far (a keep set that ends past d = 16: top-p at or near 1), whose tens of thousands of elements in one open bin no window
-// list holds (such a row took the exact path: 460 us at V = 50257).
+// Histogram bins of d = z_max - z: 1/32 wide to d = 16 (bin 512), then 1/6 wide; the last one (from d = 37.2) is open. Most
+// rows' cuts lie in the fine bins; the wide ones spread the tail of a row whose logits range far (a keep set that ends past
+// d = 16: top-p at or near 1), whose tens of thousands of elements in one open bin no window list holds (such a row took the
+// exact path: 460 us at V = 50257). Past d = 37 the whole vocabulary weighs below 2e-10. With 512 bins, 1/8 wide from d = 12
+// on, cuts at 12 to 16 listed four times as many elements: N(0, 2.5^2) rows at top-p 0.999, 256 of 151936 f32 183 us or, with
+// a row past the lists, 2450, 512 of 262144 bf16 9400 us (64 % of their rows on the exact path); with these 156-188 and 570
+// us. The 128 bins more cost flat rows 1 % (16 rows of 32000 47.4 -> 48.3 us).
 constexpr float BSC = 32.0f;    // fine bins per unit of d
-constexpr int BPT = DNB / MT;   // planner: bins per thread (contiguous)
-constexpr int WLC = 1024;       // window elements a slice gathers in LDS before one global reservation (the histogram's space)
-static_assert(BPT * MT == DNB, "");
+constexpr int BPT = (DNB + MT - 1) / MT;  // planner: bins per thread (contiguous; the last threads have none)
+constexpr int WLC = 2 * DNB;    // window elements a slice gathers in LDS before one global reservation (the histogram's space)
 
 struct DeepShared {
   HistTab h;                    // the slice's history tables while streaming
@@ -58,9 +60,9 @@ struct DeepShared {
   uint64_t pub[6];
 };
 
-// The fractional bin of a distance t = d BSC: the least of the three widths' lines, monotone in t.
+// The fractional bin of a distance t = d BSC: the lesser of the two widths' lines, monotone in t.
 __device__ __forceinline__ float bin_of(float t) {
-  return fminf(fminf(t, fmaf(t, 0.25f, 288.0f)), fminf(fmaf(t, 0.0625f, 408.0f), (float)(DNB - 1)));
+  return fminf(fminf(t, fmaf(t, 0.1875f, 416.0f)), (float)(DNB - 1));
 }
 // Bin of z (z > -inf, z <= M): monotone non-increasing in z.
 __device__ __forceinline__ uint32_t dbin(float z, float M) { return (uint32_t)bin_of((M - z) * BSC); }
@@ -191,198 +193,16 @@ __device__ __forceinline__ DGeom deep_geom(const ScanArgs &a, int nd) {
 
 // The plan of a row from its histogram (added by every slice of this launch), into the row's slot: {w2lo, w2hi, w1lo,
 // w1hi, status} and the element counts of the regions outside the windows. Run by the whole workgroup of the row's
-// last count slice: thread t holds bins 2t and 2t + 1; inclusive prefixes by block scans (wave scans, then the wave
+// last count slice: thread t holds BPT bins; inclusive prefixes by block scans (wave scans, then the wave
 // totals in order), "first bin with" queries by LDS minima, and lookups at the window edges from LDS tables.
 struct PlanShared {
   uint64_t ph[DNB], po[DNB];  // inclusive prefixes through each bin: masses in 2^-40 and 2^-64 units
-  uint32_t pc[DNB];           // and element counts (a row has fewer than 2^32 elements)
+  uint32_t pc[4];             // element counts through the windows' edges (a table of them would cost a workgroup per CU)
   uint64_t wt[3][NWV];                 // wave totals
   uint32_t q[8];                       // queries: first / last bins
 };
 
 enum { PQ_B0, PQ_B1, PQ_B2, PQ_B5, PQ_B6, PQ_B3, PQ_B4, PQ_N };
-
-__device__ __forceinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int mode, PlanShared &sh) {
-  const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
-  const gse_row &P = ds->P;
-  const float M = ds->M;
-  const uint64_t K = P.top_k > 0 ? (uint64_t)P.top_k : ~0ull;
-  const double top_p = P.top_p, min_p = P.min_p, u = ds->u;
-  uint64_t c[BPT], mh[BPT], mo[BPT];
-#pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    c[j] = ld_ag(&gh[tid * BPT + j]);
-    mh[j] = ld_ag(&gh[DNB + tid * BPT + j]);
-    mo[j] = ld_ag(&gh[2 * DNB + tid * BPT + j]);
-  }
-  // min-p keeps exp(z - M) >= min_p, i.e. d <= -ln(min_p): bins below bmlo are all kept, bins above bmhi all cut (an
-  // element's bin and -ln(min_p) are each off by less than 1e-4 bins: fp32 roundings of d BSC <= 1648)
-  const bool mp = min_p > 0.0;
-  uint32_t bmlo = 0, bmhi = 0;
-  if (mp) {
-    const float t = (float)fmin(-log(min_p) * (double)BSC, 1e6);
-    bmlo = (uint32_t)fmaxf(bin_of(t) - 0.01f, 0.0f);
-    bmhi = min((uint32_t)(bin_of(t) + 0.01f), (uint32_t)(DNB - 1));
-  }
-  // inclusive prefixes through each bin: counts, exact masses (2^-40 and 2^-64 parts) and their fp64 values
-  uint64_t cl = 0, hl = 0, ol = 0;
-#pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    cl += c[j];
-    hl += mh[j];
-    ol += mo[j];
-  }
-  const uint64_t ci = wave_incl_scan_u64(cl), hi = wave_incl_scan_u64(hl), oi = wave_incl_scan_u64(ol);
-  if (lane == WAVE - 1) {
-    sh.wt[0][w] = ci;
-    sh.wt[1][w] = hi;
-    sh.wt[2][w] = oi;
-  }
-  if (tid < PQ_N) sh.q[tid] = (tid == PQ_B5) ? 0u : (uint32_t)(DNB - 1);
-  __syncthreads();
-  uint64_t bc = 0, bh = 0, bo = 0, ctot = 0, htot = 0, otot = 0;
-#pragma unroll
-  for (int k = 0; k < NWV; ++k) {
-    const uint64_t x0 = sh.wt[0][k], x1 = sh.wt[1][k], x2 = sh.wt[2][k];
-    if (k < w) {
-      bc += x0;
-      bh += x1;
-      bo += x2;
-    }
-    ctot += x0;
-    htot += x1;
-    otot += x2;
-  }
-  uint64_t pc[BPT];
-  double pm[BPT];
-  {
-    uint64_t rc = bc + ci - cl, rh = bh + hi - hl, ro = bo + oi - ol;
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-      rc += c[j];
-      rh += mh[j];
-      ro += mo[j];
-      pc[j] = rc;
-      pm[j] = fx_val(Fx{rh, ro});
-      sh.pc[tid * BPT + j] = (uint32_t)rc;
-      sh.ph[tid * BPT + j] = rh;
-      sh.po[tid * BPT + j] = ro;
-    }
-  }
-  const double S = fx_val(Fx{htot, otot});
-  // the masses are exact; the margin covers the fp64 roundings of their values here (the finish decides exactly)
-  const double delta = 1e-12 * S;
-  const double tS = top_p * S;
-  // the windows of the cuts:
-  //   b0, b1: first bins with inclusive mass >= tS - delta, >= tS + delta (top-p: the bin of the last kept element)
-  //   b2:     first bin with inclusive count >= K (top-k: the bin of rank K - 1)
-  //   b5 - 1: last non-empty bin below bmlo (min-p: all kept, so the last element it keeps is there or after it)
-  //   b6:     first non-empty bin above bmhi (min-p: all cut)
-  {
-    uint32_t b0 = DNB - 1, b1 = DNB - 1, b2 = DNB - 1, b5 = 0, b6 = DNB - 1;
-#pragma unroll
-    for (int j = BPT - 1; j >= 0; --j) {
-      const uint32_t b = tid * BPT + j;
-      if (pm[j] >= tS - delta) b0 = b;
-      if (pm[j] >= tS + delta) b1 = b;
-      if (pc[j] >= K) b2 = b;
-      if (mp && c[j] && b > bmhi) b6 = b;
-    }
-    if (mp) {
-#pragma unroll
-      for (int j = 0; j < BPT; ++j) {
-        const uint32_t b = tid * BPT + j;
-        if (c[j] && b < bmlo) b5 = b + 1;
-      }
-    }
-    b0 = wave_min_u32(b0);
-    b1 = wave_min_u32(b1);
-    b2 = wave_min_u32(b2);
-    b5 = wave_max_u32(b5);
-    b6 = wave_min_u32(b6);
-    if (lane == 0) {
-      atomicMin(&sh.q[PQ_B0], b0);
-      atomicMin(&sh.q[PQ_B1], b1);
-      atomicMin(&sh.q[PQ_B2], b2);
-      atomicMax(&sh.q[PQ_B5], b5);
-      atomicMin(&sh.q[PQ_B6], b6);
-    }
-  }
-  __syncthreads();
-  uint32_t w1lo = sh.q[PQ_B0], w1hi = sh.q[PQ_B1];
-  if (K < ctot) {
-    w1lo = min(w1lo, sh.q[PQ_B2]);
-    w1hi = min(w1hi, sh.q[PQ_B2]);
-  }
-  if (mp) {
-    // The first cut element comes at or before each cut's own: in the window that ends where the earlier cut is sure. A
-    // window that ends before min-p's first sure cut (hi) ends in a bin by which top-p or top-k has cut. (A window from
-    // the one cut to the other held more elements than the list in flat rows, and 40 % of the C3 batches of other seeds
-    // had such a row on the exact path: 0.9 - 3.8 ms a call where 115 us is usual.)
-    const uint32_t b5 = sh.q[PQ_B5], lo = b5 ? b5 - 1u : 0u, hi = sh.q[PQ_B6];
-    w1lo = min(w1lo, lo);
-    w1hi = min(w1hi, hi);
-  }
-  // A sampled row that keeps everything (c_last = S) needs no cut window. (The exact prefix test of sampling.py:80 with
-  // top_p = 1 cuts elements whose whole remaining mass is below 2^-53 S: c_last is S within that rounding.)
-  const bool all = mode == MODE_SAMPLE && top_p >= 1.0 && K >= ctot && !mp;
-  if (all) w1lo = w1hi = DNB - 1;
-  auto at = [&](const auto *t, int b) { return b < 0 ? decltype(t[0])(0) : t[b]; };
-  // masses before w1lo and through w1hi, then the windows of the draw
-  uint32_t w2lo = w1lo, w2hi = w1hi;
-  if (mode == MODE_SAMPLE) {
-    // c_last lies between the masses through the bins at the cut window's edges (pm of those bins)
-    const double qd0 = all ? S : fx_val(Fx{at(sh.ph, (int)w1lo - 1), at(sh.po, (int)w1lo - 1)});
-    const double qd1 = all ? S : fx_val(Fx{at(sh.ph, (int)w1hi), at(sh.po, (int)w1hi)});
-    const double tlo = u * (qd0 - delta) - delta, thi = u * (qd1 + delta) + delta;
-    uint32_t b3 = DNB - 1, b4 = DNB - 1;
-#pragma unroll
-    for (int j = BPT - 1; j >= 0; --j) {
-      if (pm[j] >= tlo) b3 = tid * BPT + j;
-      if (pm[j] >= thi) b4 = tid * BPT + j;
-    }
-    b3 = wave_min_u32(b3);
-    b4 = wave_min_u32(b4);
-    if (lane == 0) {
-      atomicMin(&sh.q[PQ_B3], b3);
-      atomicMin(&sh.q[PQ_B4], b4);
-    }
-    __syncthreads();
-    w2hi = min(sh.q[PQ_B4], w1hi);
-    w2lo = min(sh.q[PQ_B3], w2hi);
-  }
-  if (all) {  // the draw's window only
-    w1lo = w2lo;
-    w1hi = w2hi;
-  } else if (w2hi + 1 >= w1lo) {  // touching or overlapping windows: one window
-    w2lo = min(w2lo, w1lo);
-    w2hi = max(w2hi, w1hi);
-    w1lo = w2lo;
-    w1hi = w2hi;
-  }
-  if (tid == 0) {
-    // the regions outside the windows from the prefixes at their edges: before the draw window (0), between the
-    // windows (1), after the cut window (counts), and the rest of the mass (2)
-    const bool sep = w1lo > w2hi + 1;
-    const uint64_t n0 = at(sh.pc, (int)w2lo - 1);
-    const uint64_t n1 = sep ? (uint64_t)(at(sh.pc, (int)w1lo - 1) - at(sh.pc, (int)w2hi)) : 0ull;
-    const uint64_t n2 = ctot - at(sh.pc, (int)w1hi);
-    const uint64_t inw = ctot - n0 - n1 - n2;
-    const uint64_t x0h = at(sh.ph, (int)w2lo - 1), x0o = at(sh.po, (int)w2lo - 1);
-    const uint64_t x1h = sep ? at(sh.ph, (int)w1lo - 1) - at(sh.ph, (int)w2hi) : 0ull;
-    const uint64_t x1o = sep ? at(sh.po, (int)w1lo - 1) - at(sh.po, (int)w2hi) : 0ull;
-    const uint64_t xm[6] = {x0h, x0o, x1h, x1o, htot - x0h - x1h, otot - x0o - x1o};
-    const uint32_t status =
-        (inw > 0 && inw <= (uint64_t)DCAP && S > 0.0 && fabsf(M) < INFINITY) ? (all ? DS_ALL : DS_PLANNED) : DS_FAIL;
-    // the region counts and sums (read by the finish, which comes after this workgroup's pick ticket and so after
-    // these stores), then the status and windows in one word, which the row's pick slices wait for
-    st_ag(&ds->acc[DA_C0], n0);  // (the element counts of the regions the pick pass sums without listing)
-    st_ag(&ds->acc[DA_C1], n1);
-    st_ag(&ds->acc[DA_C2], n2);
-    for (int k = 0; k < 6; ++k) st_ag(&ds->acc[DA_X0HI + k], xm[k]);
-    st_ag(&ds->plan, plan_word(status, w2lo, w2hi, w1lo, w1hi));
-  }
-}
 
 // ---------------------------------------------------------------------------------------------------------------------
 // Pass 2: exact masses, window list, finish.
@@ -1349,6 +1169,204 @@ __device__ __noinline__ void exact_rows(bool scan) {
   }
 }
 
+// (described at PlanShared; out of line, its LDS accessed directly: inlined it takes 11 more spilled registers)
+__device__ __noinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int mode) {
+  PlanShared &sh = g_lds.p.p.pl;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+  const gse_row &P = ds->P;
+  const float M = ds->M;
+  const uint64_t K = P.top_k > 0 ? (uint64_t)P.top_k : ~0ull;
+  const double top_p = P.top_p, min_p = P.min_p, u = ds->u;
+  uint64_t c[BPT], mh[BPT], mo[BPT];
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) {
+    const int b = min(tid * BPT + j, DNB - 1);
+    const uint64_t own = tid * BPT + j < DNB ? ~0ull : 0ull;  // (past the last bin: empty ones)
+    c[j] = ld_ag(&gh[b]) & own;
+    mh[j] = ld_ag(&gh[DNB + b]) & own;
+    mo[j] = ld_ag(&gh[2 * DNB + b]) & own;
+  }
+  // min-p keeps exp(z - M) >= min_p, i.e. d <= -ln(min_p): bins below bmlo are all kept, bins above bmhi all cut (an
+  // element's bin and -ln(min_p) are each off by less than 1e-4 bins: fp32 roundings of d BSC <= 1192)
+  const bool mp = min_p > 0.0;
+  uint32_t bmlo = 0, bmhi = 0;
+  if (mp) {
+    const float t = (float)fmin(-log(min_p) * (double)BSC, 1e6);
+    bmlo = (uint32_t)fmaxf(bin_of(t) - 0.01f, 0.0f);
+    bmhi = min((uint32_t)(bin_of(t) + 0.01f), (uint32_t)(DNB - 1));
+  }
+  // inclusive prefixes through each bin: counts, exact masses (2^-40 and 2^-64 parts) and their fp64 values
+  uint64_t cl = 0, hl = 0, ol = 0;
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) {
+    cl += c[j];
+    hl += mh[j];
+    ol += mo[j];
+  }
+  const uint64_t ci = wave_incl_scan_u64(cl), hi = wave_incl_scan_u64(hl), oi = wave_incl_scan_u64(ol);
+  if (lane == WAVE - 1) {
+    sh.wt[0][w] = ci;
+    sh.wt[1][w] = hi;
+    sh.wt[2][w] = oi;
+  }
+  if (tid < PQ_N) sh.q[tid] = (tid == PQ_B5) ? 0u : (uint32_t)(DNB - 1);
+  if (tid < 4) sh.pc[tid] = 0;  // (the count before bin 0)
+  __syncthreads();
+  uint64_t bc = 0, bh = 0, bo = 0, ctot = 0, htot = 0, otot = 0;
+#pragma unroll
+  for (int k = 0; k < NWV; ++k) {
+    const uint64_t x0 = sh.wt[0][k], x1 = sh.wt[1][k], x2 = sh.wt[2][k];
+    if (k < w) {
+      bc += x0;
+      bh += x1;
+      bo += x2;
+    }
+    ctot += x0;
+    htot += x1;
+    otot += x2;
+  }
+  uint64_t pc[BPT];
+  double pm[BPT];
+  {
+    uint64_t rc = bc + ci - cl, rh = bh + hi - hl, ro = bo + oi - ol;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+      rc += c[j];
+      rh += mh[j];
+      ro += mo[j];
+      pc[j] = rc;
+      pm[j] = fx_val(Fx{rh, ro});
+      if (tid * BPT + j < DNB) {
+        sh.ph[tid * BPT + j] = rh;
+        sh.po[tid * BPT + j] = ro;
+      }
+    }
+  }
+  const double S = fx_val(Fx{htot, otot});
+  // the masses are exact; the margin covers the fp64 roundings of their values here (the finish decides exactly)
+  const double delta = 1e-12 * S;
+  const double tS = top_p * S;
+  // the windows of the cuts:
+  //   b0, b1: first bins with inclusive mass >= tS - delta, >= tS + delta (top-p: the bin of the last kept element)
+  //   b2:     first bin with inclusive count >= K (top-k: the bin of rank K - 1)
+  //   b5 - 1: last non-empty bin below bmlo (min-p: all kept, so the last element it keeps is there or after it)
+  //   b6:     first non-empty bin above bmhi (min-p: all cut)
+  {
+    uint32_t b0 = DNB - 1, b1 = DNB - 1, b2 = DNB - 1, b5 = 0, b6 = DNB - 1;
+#pragma unroll
+    for (int j = BPT - 1; j >= 0; --j) {
+      const uint32_t b = tid * BPT + j;
+      if (pm[j] >= tS - delta) b0 = b;
+      if (pm[j] >= tS + delta) b1 = b;
+      if (pc[j] >= K) b2 = b;
+      if (mp && c[j] && b > bmhi) b6 = b;
+    }
+    if (mp) {
+#pragma unroll
+      for (int j = 0; j < BPT; ++j) {
+        const uint32_t b = tid * BPT + j;
+        if (c[j] && b < bmlo) b5 = b + 1;
+      }
+    }
+    b0 = wave_min_u32(b0);
+    b1 = wave_min_u32(b1);
+    b2 = wave_min_u32(b2);
+    b5 = wave_max_u32(b5);
+    b6 = wave_min_u32(b6);
+    if (lane == 0) {
+      atomicMin(&sh.q[PQ_B0], b0);
+      atomicMin(&sh.q[PQ_B1], b1);
+      atomicMin(&sh.q[PQ_B2], b2);
+      atomicMax(&sh.q[PQ_B5], b5);
+      atomicMin(&sh.q[PQ_B6], b6);
+    }
+  }
+  __syncthreads();
+  uint32_t w1lo = sh.q[PQ_B0], w1hi = sh.q[PQ_B1];
+  if (K < ctot) {
+    w1lo = min(w1lo, sh.q[PQ_B2]);
+    w1hi = min(w1hi, sh.q[PQ_B2]);
+  }
+  if (mp) {
+    // The first cut element comes at or before each cut's own: in the window that ends where the earlier cut is sure. A
+    // window that ends before min-p's first sure cut (hi) ends in a bin by which top-p or top-k has cut. (A window from
+    // the one cut to the other held more elements than the list in flat rows, and 40 % of the C3 batches of other seeds
+    // had such a row on the exact path: 0.9 - 3.8 ms a call where 115 us is usual.)
+    const uint32_t b5 = sh.q[PQ_B5], lo = b5 ? b5 - 1u : 0u, hi = sh.q[PQ_B6];
+    w1lo = min(w1lo, lo);
+    w1hi = min(w1hi, hi);
+  }
+  // A sampled row that keeps everything (c_last = S) needs no cut window. (The exact prefix test of sampling.py:80 with
+  // top_p = 1 cuts elements whose whole remaining mass is below 2^-53 S: c_last is S within that rounding.)
+  const bool all = mode == MODE_SAMPLE && top_p >= 1.0 && K >= ctot && !mp;
+  if (all) w1lo = w1hi = DNB - 1;
+  auto at = [&](const auto *t, int b) { return b < 0 ? decltype(t[0])(0) : t[b]; };
+  // masses before w1lo and through w1hi, then the windows of the draw
+  uint32_t w2lo = w1lo, w2hi = w1hi;
+  if (mode == MODE_SAMPLE) {
+    // c_last lies between the masses through the bins at the cut window's edges (pm of those bins)
+    const double qd0 = all ? S : fx_val(Fx{at(sh.ph, (int)w1lo - 1), at(sh.po, (int)w1lo - 1)});
+    const double qd1 = all ? S : fx_val(Fx{at(sh.ph, (int)w1hi), at(sh.po, (int)w1hi)});
+    const double tlo = u * (qd0 - delta) - delta, thi = u * (qd1 + delta) + delta;
+    uint32_t b3 = DNB - 1, b4 = DNB - 1;
+#pragma unroll
+    for (int j = BPT - 1; j >= 0; --j) {
+      if (pm[j] >= tlo) b3 = tid * BPT + j;
+      if (pm[j] >= thi) b4 = tid * BPT + j;
+    }
+    b3 = wave_min_u32(b3);
+    b4 = wave_min_u32(b4);
+    if (lane == 0) {
+      atomicMin(&sh.q[PQ_B3], b3);
+      atomicMin(&sh.q[PQ_B4], b4);
+    }
+    __syncthreads();
+    w2hi = min(sh.q[PQ_B4], w1hi);
+    w2lo = min(sh.q[PQ_B3], w2hi);
+  }
+  if (all) {  // the draw's window only
+    w1lo = w2lo;
+    w1hi = w2hi;
+  } else if (w2hi + 1 >= w1lo) {  // touching or overlapping windows: one window
+    w2lo = min(w2lo, w1lo);
+    w2hi = max(w2hi, w1hi);
+    w1lo = w2lo;
+    w1hi = w2hi;
+  }
+  // the element counts through the windows' edges
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) {
+    const uint32_t b = tid * BPT + j;
+    if (b + 1u == w2lo) sh.pc[0] = (uint32_t)pc[j];
+    if (b == w2hi) sh.pc[1] = (uint32_t)pc[j];
+    if (b + 1u == w1lo) sh.pc[2] = (uint32_t)pc[j];
+    if (b == w1hi) sh.pc[3] = (uint32_t)pc[j];
+  }
+  __syncthreads();
+  if (tid == 0) {
+    // the regions outside the windows from the prefixes at their edges: before the draw window (0), between the
+    // windows (1), after the cut window (counts), and the rest of the mass (2)
+    const bool sep = w1lo > w2hi + 1;
+    const uint64_t n0 = sh.pc[0];
+    const uint64_t n1 = sep ? (uint64_t)(sh.pc[2] - sh.pc[1]) : 0ull;
+    const uint64_t n2 = ctot - sh.pc[3];
+    const uint64_t inw = ctot - n0 - n1 - n2;
+    const uint64_t x0h = at(sh.ph, (int)w2lo - 1), x0o = at(sh.po, (int)w2lo - 1);
+    const uint64_t x1h = sep ? at(sh.ph, (int)w1lo - 1) - at(sh.ph, (int)w2hi) : 0ull;
+    const uint64_t x1o = sep ? at(sh.po, (int)w1lo - 1) - at(sh.po, (int)w2hi) : 0ull;
+    const uint64_t xm[6] = {x0h, x0o, x1h, x1o, htot - x0h - x1h, otot - x0o - x1o};
+    const uint32_t status =
+        (inw > 0 && inw <= (uint64_t)DCAP && S > 0.0 && fabsf(M) < INFINITY) ? (all ? DS_ALL : DS_PLANNED) : DS_FAIL;
+    // the region counts and sums (read by the finish, which comes after this workgroup's pick ticket and so after
+    // these stores), then the status and windows in one word, which the row's pick slices wait for
+    st_ag(&ds->acc[DA_C0], n0);  // (the element counts of the regions the pick pass sums without listing)
+    st_ag(&ds->acc[DA_C1], n1);
+    st_ag(&ds->acc[DA_C2], n2);
+    for (int k = 0; k < 6; ++k) st_ag(&ds->acc[DA_X0HI + k], xm[k]);
+    st_ag(&ds->plan, plan_word(status, w2lo, w2hi, w1lo, w1hi));
+  }
+}
+
 // A verify node that takes dist + mss wants dist's keep boundary, not a draw.
 __device__ __forceinline__ int row_mode(const ScanArgs &a, const gse_row &P) {
   return a.tree && (P.flags & GSE_ROW_MSS) ? (int)MODE_DIST : a.mode;
@@ -1398,7 +1416,7 @@ __device__ __forceinline__ void count_item(const ScanArgs &a, int slot, int slic
   __syncthreads();  // (every thread has read the ticket: the plan's tables reuse the slice's LDS)
   if (!lastc) return;
   __builtin_amdgcn_s_setprio(3);  // (the row's other slices wait for the plan)
-  plan_block(gh, ds, row_mode(a, P), ps.p.pl);
+  plan_block(gh, ds, row_mode(a, P));
   if (tid == 0) {
     ds->cdone = 0u;
     g_pl[slot >> 6] |= 1ull << (slot & 63);  // (its pick item takes the rows-planned ticket)

@@ -98,7 +98,7 @@ static_assert(sizeof(SliceRec) == 64, "");
 constexpr int DEEP_MAX = 1024;  // split-row slots at most (a handle has min(max_rows, DEEP_MAX); more deep rows: the
                                 // exact path takes them)
 constexpr int DSMAX = 64;      // slices per deep row, at most
-constexpr int DNB = 512;       // histogram bins of d = z_max - z: 1/32 wide to d = 12, then wider (gse_deep.hip)
+constexpr int DNB = 640;       // histogram bins of d = z_max - z: 1/32 wide to d = 16, then wider (gse_deep.hip)
 constexpr int DCAP = 8192;     // window elements listed per deep row
 
 // DS_ALL: planned, and every element is kept (a sampled row with no top-p, top-k or min-p cut): the list holds the draw's

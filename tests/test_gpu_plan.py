@@ -54,6 +54,26 @@ def test_keep_all_and_long_tails(ge, gpu, v):
     assert (paths == ge._lib.PATH_DEEP).sum() > 0
 
 
+@pytest.mark.parametrize("n,v,dtype", [(512, 262144, "bf16"), (256, 151936, "f32")])
+def test_cuts_far_below_the_maximum(ge, gpu, n, v, dtype):
+    """Large batches of wide flat rows whose top-p cut lies 12 to 16 below the maximum (slices of 64K tokens: what one
+    slice lists of a window must fit its LDS list): all of them on the split-row pass, tokens of every 32nd row against
+    the oracle."""
+    g = torch.Generator(device=gpu).manual_seed(v)
+    x = torch.randn((n, v), generator=g, device=gpu).mul_(2.5)
+    x = x.bfloat16() if dtype == "bf16" else x
+    P = ge.sampling.SamplingParams
+    params = [P(temperature=1.0, top_p=[0.998, 0.999, 0.9995][r % 3]) for r in range(n)]
+    u = np.random.default_rng(v).random(n)
+    sel = ge.sampling.sample_ex(x, params, None, None, None, uniforms=u)
+    paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
+    assert (paths == ge._lib.PATH_EXACT).sum() == 0, (paths == ge._lib.PATH_EXACT).sum()
+    assert (paths == ge._lib.PATH_DEEP).sum() > n // 2
+    some = list(range(0, n, 32))
+    want = ora.sample(x[some].float().cpu().numpy(), [params[r] for r in some], None, None, None, uniforms=u[some])
+    assert [sel.tolist()[r] for r in some] == want
+
+
 def test_dist_of_long_tails(ge, gpu):
     """dist over such rows: every probability against the oracle's."""
     rng = np.random.default_rng(4)
