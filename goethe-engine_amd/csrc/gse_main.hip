@@ -119,8 +119,12 @@ __device__ __forceinline__ void set_hard(const ScanArgs &a, RowInfo *ri, uint64_
 enum { EV_DONE = 0, EV_HARD = 1 };
 // The least share of the mass that top-p keeps that the head must hold for the row's draw to be looked for in it. In a
 // flatter row few draws fall there, and a batch of such rows needs the split-row pass for the others anyway: skipping
-// their sort and evaluation keeps the main pass's tail short.
-constexpr double HEAD_DRAW = 0.25;
+// their sort and evaluation keeps the main pass's tail short. A verify round's sampled rows are many and alike: a larger
+// share (8 chains of 7 bf16 nodes over 12574 tokens at top-p 0.95 73.8 -> 70.6 us, 2 trees of 32000 217 -> 213, 32 chains of
+// 32000 89.8 -> 88.1; with 0.75 for sampled batches too, one flat f32 row of 128256 38 -> 45 us, 24 mixed rows of 50257 43 ->
+// 49).
+constexpr double HEAD_DRAW = 0.25, HEAD_DRAW_TREE = 0.75;
+__device__ __forceinline__ double head_draw(const ScanArgs &a) { return a.tree ? HEAD_DRAW_TREE : HEAD_DRAW; }
 constexpr uint32_t NONE = 0xFFFFFFFFu;
 
 struct RowEval {
@@ -248,7 +252,7 @@ __device__ __forceinline__ int evaluate(const RowEval &ev, const uint64_t *arr, 
     // (top-p the only cut) top_p S; at most the prefix of the first that surely fails, or top_p S and one element more
     // (the last kept one, at most the head's last), or S. Only a token is wanted: dist and verify nodes that take
     // dist + mss need the boundary itself. (m1 = 0: the bound exceeds S, so even rank 0 may fail, and no prefix comes before)
-    if (n == 0 || m1 == 0 || a.mode != MODE_SAMPLE || (a.tree && (P.flags & GSE_ROW_MSS)) || htot < HEAD_DRAW * topp * Sm)
+    if (n == 0 || m1 == 0 || a.mode != MODE_SAMPLE || (a.tree && (P.flags & GSE_ROW_MSS)) || htot < head_draw(a) * topp * Sm)
       return EV_HARD;
     const double clo = m1 != NONE ? ee[m1 - 1] : P.top_k > 0 || minp > 0.0 ? htot : fmax(htot, tlo);
     const double chi = m2 != NONE ? ee[m2 - 1] : fmin(Sm + B, thi + (n > 1 ? ee[n - 1] - ee[n - 2] : htot));
@@ -583,7 +587,7 @@ __device__ __forceinline__ void resolve_row(const ScanArgs &a, int row, const gs
       const double B = ev.B + 2e-15 * (ev.S + hhi);
       past = hhi < P.top_p * (ev.S + hlo - B);
       // (unless the draw surely falls inside the head: c_last is at most S, and top_p S and one unlisted element)
-      if (past && a.mode == MODE_SAMPLE && !(a.tree && (P.flags & GSE_ROW_MSS)) && h >= HEAD_DRAW * P.top_p * (ev.S + h)) {
+      if (past && a.mode == MODE_SAMPLE && !(a.tree && (P.flags & GSE_ROW_MSS)) && h >= head_draw(a) * P.top_p * (ev.S + h)) {
         const double u = a.uni ? a.uni[row] : uniform64(P.seed, P.idx);
         const double ek = exp_nonpos((double)fkey_inv(kappa) - M, sh.etab), Sh = ev.S + hhi + B;
         past = !(u * fmin(Sh, P.top_p * Sh + ek) < hlo);
