@@ -208,4 +208,7 @@ def test_window_lists_of_ties(ge, gpu, v, flags):
     for x in (torch.from_numpy(base).bfloat16(), torch.from_numpy(np.round(base * 16) / 16),
               torch.from_numpy(np.round(base * 64) / 64)):
         sel = ge.sampling.sample_ex(x.to(gpu), params, None, None, None, uniforms=u, flags=flags)
+        paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
         assert sel.tolist() == ora.sample(x.float().numpy(), params, None, None, None, uniforms=u)
+        # (a finish that fails its checks hands its row to the exact path, which would hide it)
+        assert (paths == ge._lib.PATH_DEEP).any() and not (paths == ge._lib.PATH_EXACT).any(), paths
