@@ -37,7 +37,7 @@ enum : uint32_t {
 
 enum { MODE_SAMPLE = 0, MODE_DIST = 1 };
 
-constexpr int CH = 8192;  // tokens per slice (the exact path, dist, and the verify and pick passes walk rows in these)
+constexpr int CH = 8192;  // tokens per slice (the exact path and the verify passes walk rows in these)
 // gse_sample_noalloc's static workspace: batches of at most this many rows of at most this many tokens.
 constexpr uint32_t NOALLOC_ROWS = 32;
 constexpr uint32_t NOALLOC_VOCAB = 163840;

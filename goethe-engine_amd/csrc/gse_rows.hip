@@ -270,8 +270,8 @@ __device__ __forceinline__ MssTok<D> mss_load(const double *p, const MssKid (&k)
 
 // The kids past level MSS_LEVELS, by one workgroup, in place in p: the residual of the level before (written by this
 // workgroup), total its sum. A kid is one pass over the row: the division by the sum before, the residual, and the slices'
-// sums, which the next test and the draw use (a residual that is not divided draws the same), with 16 tokens a thread in
-// flight. Bound by the chain of one workgroup's slices. Every kid rejected, us a call:
+// sums, which the next test and the draw use (a residual that is not divided draws the same), eight tokens a
+// thread loading at a time. Bound by the chain of one workgroup's slices. Every kid rejected, us a call:
 //   16 nodes of 128256: 4 kids 517, 16 kids 3070 (two passes a kid of 256 tokens at a time and a third for the draw: 819,
 //   5700; one workgroup of 1024 threads a node over contiguous runs: 1823, 6790)
 //   64 nodes of 151936: 4 kids 1240, 16 kids 8110, one-hot 850, 5150 (1840, 13400, 1410, 8720; 3380, 12600, 2700, 9860)

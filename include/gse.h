@@ -8,7 +8,10 @@
  *   Structs     every in/out struct starts with `size`, the caller's sizeof; the library reads only fields inside
  *               min(size, its own size) and treats absent fields as zero.
  *   Handles     gse_open returns an independent instance (own device workspace). One handle is not thread safe; each
- *               call takes the caller's HIP stream and is asynchronous on it.
+ *               call takes the caller's HIP stream and is asynchronous on it. Every call that launches work but
+ *               gse_pack_mask uses the handle's workspace (gse_draw, gse_mss, gse_draft_pick and gse_qprob keep their
+ *               partial sums and tickets there too): calls of one handle must not overlap on the device. Use one handle
+ *               per stream, or order the streams. Captured calls count as calls of the stream that replays them.
  *   Errors      functions return GSE_OK (0) or a negative GSE_E_* code; gse_last_error(h) returns the text of the last
  *               error on that handle (gse_last_error(NULL): the last gse_open failure on this thread).
  *   Memory      every data pointer below is a device pointer unless marked host. Inputs are borrowed, never written;
@@ -109,7 +112,8 @@ enum {
                             * (same results). For batches that cannot use it, to save its launch: greedy rows of
                             * gse_sample never do (the Python layer sets it when every row is greedy). Since ABI 1.3. */
   GSE_BATCH_SUBBIN_FINISH = 16u /* testing: the split-row finish of every row takes its sub-bin walk, which it otherwise
-                                 * keeps for window lists longer than 2048 entries (same results). Since ABI 1.4. */
+                                 * keeps for window lists longer than 2048 entries or crowded with ties (same results).
+                                 * Since ABI 1.4. */
 };
 
 typedef struct gse_out {
@@ -250,8 +254,7 @@ GSE_API int gse_dist(gse_handle *h, const gse_batch *in, double *probs, int64_t 
  * strict node, spec.py:88-103) with one call that runs every node of every request on the device and walks the trees
  * there: no host round trip per level. Stop rules (engine.py:218-229) stay with the caller, which ends each emitted
  * sequence at its first stop reason; the tokens before it do not depend on what follows. in->rows are the tree nodes.
- * With drafter logits, the q rows' statistics run on a stream of the handle, forked from in->stream at the call's start
- * and joined back before they are used: the call stays ordered on in->stream like every other. */
+ * With drafter logits, the q rows' statistics are part of the call's own launches: everything runs on in->stream. */
 GSE_API int gse_verify_tree(gse_handle *h, const gse_batch *in, const gse_tree *tree, const gse_tree_out *out);
 
 /* Replaces: goethe_engine/spec.py:151-159 TreeDrafter._pick (torch.sort / softmax / draw on the host) for a batch of

@@ -164,6 +164,42 @@ def test_rows_past_the_handles_size(ge, gpu):
     h.close()
 
 
+def test_two_streams_with_a_handle_each(ge, gpu):
+    """draw, mss and qprob keep their partial sums in the handle's workspace: calls that overlap on two streams, each with
+    its own handle (which the Python layer keeps per stream), do not disturb each other."""
+    v, n = 128256, 8
+    rng = np.random.default_rng(5)
+    streams = [torch.cuda.Stream(gpu) for _ in range(2)]
+    data = []
+    for s in range(2):
+        q, u = rng.random((n, v)), rng.random(n)
+        p, kids = _nodes(v, n, rng)
+        x = torch.from_numpy(rng.normal(size=(n, v)).astype(np.float32))
+        want = ([ora.draw(q[r], u[r]) for r in range(n)], [spo.mss(p[a], kids[a], a, s) for a in range(n)])
+        data.append((torch.from_numpy(q).to(gpu), torch.from_numpy(u).to(gpu), torch.from_numpy(p).to(gpu), kids,
+                     x.to(gpu), torch.softmax(x.double() / 0.7, 1).numpy(), want))
+    torch.cuda.synchronize()
+    lib = ge._lib
+    for _ in range(3):
+        outs = []
+        for s in range(2):
+            with torch.cuda.stream(streams[s]):
+                q, u, p, kids, x, _, _ = data[s]
+                h = lib.handle(gpu.index, n, v)
+                out = torch.full((6, n), -7, dtype=torch.int32, device=gpu)
+                for k in range(6):
+                    h.call("gse_draw", q.data_ptr(), v, n, v, u.data_ptr(), out[k].data_ptr(), lib.stream_of(gpu.index))
+                outs.append((h, out, ge.spec.qprob(x, 0.7)))
+        assert outs[0][0] is not outs[1][0]
+        for s in range(2):
+            with torch.cuda.stream(streams[s]):
+                _, _, p, kids, _, sm, want = data[s]
+                toks, ks = ge.spec.mss_batch(p, kids, list(range(n)), [s] * n)
+                assert list(zip(toks, ks)) == want[1]
+                assert outs[s][1].cpu().tolist() == [want[0]] * 6
+                np.testing.assert_allclose(outs[s][2].cpu().numpy(), sm, rtol=1e-13)
+
+
 def test_rows_of_nearly_2_31_tokens(ge, gpu):
     """The last slice of a row of 2^31 - 1 tokens reaches past 2^31: draw and qprob read and write inside the row, and a
     longer row is refused."""
