@@ -588,7 +588,7 @@ __device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared
 // and one block minimum each. The unlisted region between the windows (X1, c1 elements) counts before the cut
 // window's entries. The tests and fixed-point sums are finish_row's; a failed check leaves the row to the exact path.
 constexpr int FB = 1024;  // key buckets per window
-constexpr int FBK = 64;   // the largest bucket whose members are ranked by counting
+constexpr int FBK = 1024; // the most bucket members that a thread reads to rank its entries by counting
 static_assert(2 * 2 * FB * sizeof(uint32_t) <= SUBC * sizeof(uint64_t), "bucket counts and starts live in sub");
 static_assert(SUBC >= LC, "masses by rank live in sub");
 
@@ -928,10 +928,13 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   }
   __syncthreads();
   const uint32_t n0 = sep ? bofs[FB] : (uint32_t)n;  // entries of the draw window (they rank first)
-  // A crowded bucket (a tie group: bf16 logits) goes to the sub-bin walk, which sorts only the groups that hold the cut and
-  // the draw: ranking its members against each other reads them all once per member (one bf16 row of 151936 tokens: 67
-  // us; sorting the whole list in registers 66; the walk 61).
-  if (sh.q[2] > (uint32_t)FBK) return 1;
+  // A thread reads the bucket of each of its entries, one after the other: the largest bucket times the entries a thread.
+  // Past FBK (a large tie group: bf16 logits) the list goes to the sub-bin walk, which sorts only the groups that hold the
+  // cut and the draw (one bf16 row of 151936 tokens: counting 67 us, sorting the whole list in registers 66, the walk 61).
+  // Below, the walk's passes cost more than the counting: with every bucket past 64 walked, 8 bf16 rows of 128256 took 68.5
+  // us (57.9 now), a verify round of 4 bf16 chains of 7 over 128256 128.0 (116.0), of 16 trees over 50257 202 (191). Limits of
+  // 512 and 2048: within 0.3 us, but 2 chains of 100000 86.5 at 512 (83.3) and 4 chains of 151936 149.3 at 2048 (148.3).
+  if (sh.q[2] * (uint32_t)((n + MT - 1) / MT) > (uint32_t)FBK) return 1;
 #pragma unroll
   for (int j = 0; j < SP; ++j)
     if (j * MT + tid < n) sh.lc[bofs[bucket(j)] + sl[j]] = v[j];

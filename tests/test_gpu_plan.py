@@ -212,3 +212,23 @@ def test_window_lists_of_ties(ge, gpu, v, flags):
         assert sel.tolist() == ora.sample(x.float().numpy(), params, None, None, None, uniforms=u)
         # (a finish that fails its checks hands its row to the exact path, which would hide it)
         assert (paths == ge._lib.PATH_DEEP).any() and not (paths == ge._lib.PATH_EXACT).any(), paths
+
+
+@pytest.mark.parametrize("step", [64, 16])
+def test_tie_groups_around_the_counting_limit(ge, gpu, step):
+    """Rows of tie groups of one size each, from a few members to more than the finish ranks by counting, with one to four
+    groups in a window (grid steps of 1/64 and 1/16 against bins of 1/32)."""
+    sizes = [48, 64, 65, 128, 193, 255, 256, 257, 341, 342, 511, 512, 513, 700, 1024, 1025]
+    n, v = len(sizes), 40000
+    rng = np.random.default_rng(step)
+    P = ge.sampling.SamplingParams
+    x = np.empty((n, v), np.float32)
+    for r, g in enumerate(sizes):
+        x[r] = 4.0 - (rng.permutation(v) // g).astype(np.float32) / step
+    for top_p in (0.9, 1.0):
+        params = [P(temperature=1.0, top_p=top_p) for _ in range(n)]
+        u = np.array([ora.uniform(r, 3) for r in range(n)], np.float64)
+        sel = ge.sampling.sample_ex(torch.from_numpy(x).to(gpu), params, None, None, None, uniforms=u)
+        paths = ge._lib.handle(gpu.index, n, v).row_paths(n)
+        assert sel.tolist() == ora.sample(x, params, None, None, None, uniforms=u)
+        assert (paths == ge._lib.PATH_DEEP).any() and not (paths == ge._lib.PATH_EXACT).any(), paths
