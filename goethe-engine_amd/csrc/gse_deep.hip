@@ -289,16 +289,24 @@ __device__ __forceinline__ Fx mass_of(uint32_t key, double M, const double *etab
 }
 
 // What the finish uses of the launch arguments (by value: the kernel keeps its arguments in registers).
+// A verify node that takes dist + mss wants dist's keep boundary, not a draw.
+template <typename A>
+__device__ __forceinline__ int row_mode(const A &a, const gse_row &P) {
+  return a.tree && (P.flags & GSE_ROW_MSS) ? (int)MODE_DIST : a.mode;
+}
+
 struct FinArgs {
   const uint64_t *lst;  // the row's window list
   RowInfo *info;
   int32_t *tokens;
   int mode;
+  bool tree;
 };
 
 // (not inlined: its registers are allocated apart from the streaming code of the pick pass)
-__device__ __noinline__ void finish_row(const FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab) {
+__device__ __noinline__ void finish_row(FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab) {
   const int tid = threadIdx.x;
+  a.mode = row_mode(a, ds->P);
   const gse_row &P = ds->P;
   const int row = ds->row;
   const float Mf = ds->M;
@@ -818,7 +826,7 @@ __device__ __forceinline__ void finish_block(const FinArgs a, DeepSlot *ds, FinS
   }
 }
 
-__device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab) {
+__device__ __noinline__ int finish_sorted(FinArgs a, DeepSlot *ds, FinShared &sh, const double *etab) {
   constexpr int SP = LC / MT;  // entries (and ranks) per thread
   const int tid = threadIdx.x, w = tid >> 6;
   // every load the finish makes, issued together: the list's first LC entries (entries past its end are stale and
@@ -835,6 +843,7 @@ __device__ __noinline__ int finish_sorted(const FinArgs a, DeepSlot *ds, FinShar
   const double M = (double)Mf, u = ds->u;
   const uint64_t K = ds->P.top_k > 0 ? (uint64_t)ds->P.top_k : ~0ull;
   const double topp = ds->P.top_p, minp = ds->P.min_p;
+  a.mode = row_mode(a, ds->P);  // (one of these loads, not one before them: 0.4 us a call)
   if (spoil != 0u) return 0;  // (a slice gave up waiting for the plan: the exact path takes the row)
   if (nraw > (uint32_t)LC) return 1;
   const int n = (int)nraw;
@@ -1370,11 +1379,6 @@ __device__ __noinline__ void plan_block(const uint64_t *gh, DeepSlot *ds, int mo
   }
 }
 
-// A verify node that takes dist + mss wants dist's keep boundary, not a draw.
-__device__ __forceinline__ int row_mode(const ScanArgs &a, const gse_row &P) {
-  return a.tree && (P.flags & GSE_ROW_MSS) ? (int)MODE_DIST : a.mode;
-}
-
 template <int DT, bool AL>
 __device__ __forceinline__ void count_item(const ScanArgs &a, int slot, int slice, const DGeom &g, PickShared &ps,
                                            const double *etab) {
@@ -1529,7 +1533,7 @@ __device__ __forceinline__ void finish_item(const ScanArgs &a, int fs, PickShare
   __builtin_amdgcn_s_setprio(3);  // (the finish is the row's critical path)
   if (tid == 0) g_fin = 0u;
   if (planned) {
-    const FinArgs fa{a.dlist + (size_t)slot * DCAP, a.info, a.tokens, row_mode(a, ds->P)};
+    const FinArgs fa{a.dlist + (size_t)slot * DCAP, a.info, a.tokens, a.mode, a.tree != 0};
     if (a.fin_sorted ? finish_sorted(fa, ds, ps.f, etab) != 0 : ld_ag(&ds->spoil) == 0u) {
       finish_row(fa, ds, ps.f, etab);
     }
